@@ -345,7 +345,8 @@ int build_scene(bh_ctx* ctx, const bh_scene* sc, const bh_options* opt_in, DevSc
 // other scenes take the FP64 march.
 bool fp32_eligible(const DevScene& d) { return d.fast_ok != 0; }
 
-// FP32 march then the FP64 band kernel, or the FP64 reference march.
+// The scene record and clear queue counts, then the FP32 march and the FP64
+// band kernel, or the FP64 reference march.
 int launch_frame(bh_ctx* ctx, const DevScene& host_scene, DevScene* d_scene, const DevOut& out,
                  const DevQueue& q, hipStream_t st) {
   const int W = host_scene.W, H = host_scene.H;
@@ -355,25 +356,22 @@ int launch_frame(bh_ctx* ctx, const DevScene& host_scene, DevScene* d_scene, con
       return fail(ctx, BH_ERR_INVALID_ARG, "FP32 march launched without a band queue");
     const bool esc = host_scene.escape != 0;
     const bool sph = host_scene.n_spheres > 0;
+    HIP_TRY(ctx, bh::launch_scene(host_scene, d_scene, q.count, st));
     HIP_TRY(ctx, bh::launch_march_fp32(d_scene, out, W, H, q, st, esc, sph, host_scene.nstep));
     HIP_TRY(ctx, bh::launch_band(d_scene, out, q, st, esc, sph));
   } else {
+    HIP_TRY(ctx, bh::launch_scene(host_scene, d_scene, nullptr, st));
     HIP_TRY(ctx, bh::launch_march_fp64(d_scene, out, W, H, st));
   }
   return BH_OK;
 }
 
-// The context's FP64 queue for frames up to W x H, with zeroed count pairs
-// (the FP64 pass keeps them zeroed between frames).
+// The context's FP64 queue for frames up to W x H (each frame's first launch
+// clears its counts).
 int queue_buffers(bh_ctx* ctx, int W, int H, DevQueue* q) {
-  const bool fresh = ctx->qcount.p == nullptr;
   int rc = ensure(ctx, ctx->qitems, bh::queue_items(W, H) * sizeof(uint64_t));
   if (rc) return rc;
   if ((rc = ensure(ctx, ctx->qcount, bh::kQueueCountWords * sizeof(uint32_t)))) return rc;
-  if (fresh) {
-    HIP_TRY(ctx, bh::launch_zero_u32((uint32_t*)ctx->qcount.p, (int)bh::kQueueCountWords,
-                                     ctx->stream));
-  }
   *q = DevQueue{(uint64_t*)ctx->qitems.p, (uint32_t*)ctx->qcount.p, bh::queue_sub_cap(W, H)};
   return BH_OK;
 }
@@ -666,13 +664,16 @@ int build_diff(bh_ctx* ctx, const bh_diff_params* p, int precision, bh::DiffScen
   return BH_OK;
 }
 
-// Fused path launches: every frame's march in one launch (up to 1024 frames
-// each), then every frame's FP64 band pass in one launch.
+// Fused path launches: the queue counts cleared and every frame's march in one
+// launch (up to 1024 frames each), then every frame's FP64 band pass in one launch.
 constexpr int kFramesPerLaunch = 1024;
 
 hipError_t path_march(const bh_path* p, hipStream_t st) {
   const DevOut o{p->d_rgb, p->d_hit, nullptr, nullptr, nullptr};
   const DevQueue q{p->d_qitems, p->d_qcount, p->sub_cap};
+  const hipError_t z =
+      bh::launch_zero_u32(p->d_qcount, (int)bh::kQueueCountWords * p->n_frames, st);
+  if (z != hipSuccess) return z;
   for (int f0 = 0; f0 < p->n_frames; f0 += kFramesPerLaunch) {
     const int nf = std::min(kFramesPerLaunch, p->n_frames - f0);
     const hipError_t e = bh::launch_march_frames(p->d_scenes, o, p->W, p->H, f0, nf, q, st,
@@ -871,7 +872,6 @@ int bh_render_device(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
     if ((rc = ensure(ctx, ctx->scene, sizeof(DevScene)))) return rc;
     DevQueue q;
     if ((rc = queue_buffers(ctx, d.W, d.H, &q))) return rc;
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->scene.p, &d, sizeof d, hipMemcpyHostToDevice, ctx->stream));
     DevOut o{out_device->rgb, out_device->hit, out_device->phi_end, out_device->hit_point,
              out_device->steps};
     return launch_frame(ctx, d, (DevScene*)ctx->scene.p, o, q, ctx->stream);
@@ -895,7 +895,6 @@ int bh_render_device_noalloc(bh_ctx* ctx, const bh_scene* scene, const bh_option
                       std::to_string(bh::queue_items(d.W, d.H)) + ")");
     (void)hipSetDevice(ctx->device);
     const bh::NoallocLayout l = bh::noalloc_layout(ctx->noalloc);
-    HIP_TRY(ctx, bh::launch_noalloc_setup(d, l, ctx->stream));
     DevOut o{out_device->rgb, out_device->hit, out_device->phi_end, out_device->hit_point,
              out_device->steps};
     const DevQueue q{l.items, l.count, bh::queue_sub_cap(d.W, d.H)};
@@ -947,15 +946,15 @@ int bh_time_render(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt, in
     DevQueue q;
     if ((rc = queue_buffers(ctx, d.W, d.H, &q))) return rc;
     hipStream_t st = ctx->stream;
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->scene.p, &d, sizeof d, hipMemcpyHostToDevice, st));
     DevOut o{(uint8_t*)ctx->rgb.p, (uint8_t*)ctx->hit.p, nullptr, nullptr, nullptr};
     DevScene* ds = (DevScene*)ctx->scene.p;
     const bool fast = fp32_eligible(d);
     // warm-up
     if ((rc = launch_frame(ctx, d, ds, o, q, st))) return rc;
+    if (fast) HIP_TRY(ctx, bh::launch_zero_u32(q.count, (int)bh::kQueueCountWords, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));
-    // main kernel: iters back-to-back launches between one event pair (the
-    // queue is cleared afterwards); whole frame: iters march + band launches
+    // main kernel: iters back-to-back launches between one event pair, from
+    // clear queue counts; whole frame: iters times all its launches
     float main_ms = 0, total_ms = 0;
     std::vector<uint32_t> cnt(bh::kQueueCountWords, 0u);
     HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
@@ -970,7 +969,6 @@ int bh_time_render(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt, in
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
     if (fast) {
       HIP_TRY(ctx, hipMemcpyAsync(cnt.data(), q.count, cnt.size() * 4, hipMemcpyDeviceToHost, st));
-      HIP_TRY(ctx, bh::launch_zero_u32(q.count, (int)bh::kQueueCountWords, st));
     }
     HIP_TRY(ctx, hipEventRecord(ctx->ev2, st));
     for (int it = 0; it < iters; ++it)
@@ -1038,7 +1036,6 @@ int bh_path_create(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
     p->nstep = frames[0].nstep;
     if ((e = hipMalloc(&p->d_qitems, qitems * n_frames * sizeof(uint64_t))) != hipSuccess) return cleanup(e, "hipMalloc queue");
     if ((e = hipMalloc(&p->d_qcount, qwords * 4 * (size_t)n_frames)) != hipSuccess) return cleanup(e, "hipMalloc queue count");
-    if ((e = hipMemset(p->d_qcount, 0, qwords * 4 * (size_t)n_frames)) != hipSuccess) return cleanup(e, "hipMemset queue count");
     if ((e = hipMemcpy(p->d_scenes, frames.data(), sizeof(DevScene) * n_frames, hipMemcpyHostToDevice)) != hipSuccess)
       return cleanup(e, "hipMemcpy scenes");
     p->events.resize((size_t)n_frames + 1, nullptr);
@@ -1060,8 +1057,9 @@ int bh_path_create(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
       if (fp32_eligible(f)) {
         const bool esc = f.escape != 0;
         const bool sph = f.n_spheres > 0;
-        hipError_t le =
-            bh::launch_march_fp32(p->d_scenes + i, o, p->W, p->H, q, st, esc, sph, f.nstep);
+        hipError_t le = bh::launch_zero_u32(q.count, (int)bh::kQueueCountWords, st);
+        if (le == hipSuccess)
+          le = bh::launch_march_fp32(p->d_scenes + i, o, p->W, p->H, q, st, esc, sph, f.nstep);
         if (le == hipSuccess) le = hipEventRecord(p->events[(size_t)i], st);
         if (le == hipSuccess) le = hipStreamWaitEvent(side, p->events[(size_t)i], 0);
         if (le == hipSuccess) le = bh::launch_band(p->d_scenes + i, o, q, side, esc, sph);

@@ -149,8 +149,9 @@ struct NoallocLayout {
 // stand-in of the array's name is no device address).
 hipError_t noalloc_scratch(void** ptr);
 NoallocLayout noalloc_layout(void* base);
-// Scene record into the array, queue counts cleared; on stream.
-hipError_t launch_noalloc_setup(const DevScene& s, const NoallocLayout& l, hipStream_t stream);
+// Scene record into device memory (by a kernel argument) and the queue's
+// count words (null: none) cleared; on stream.
+hipError_t launch_scene(const DevScene& s, DevScene* dst, uint32_t* count, hipStream_t stream);
 
 // FMA issue-rate probe (bh_probe.hip): TFLOP/s of plain FMA chains in
 // precision T, 8 waves per SIMD on n_cu compute units; sink: 256 elements.

@@ -126,8 +126,7 @@ void march_frames_kernel(const DevScene* __restrict__ sp, DevOut out, DevQueue q
 // (the back of the sub-queues; blk takes part blk / kQueueSubs of sub-queue
 // blk mod kQueueSubs), the nband workgroups after them the band rays of all
 // sub-queues packed together (the front segments, indexed through their
-// prefix sum).  The last workgroup to finish clears the frame's counts for
-// the next frame; count[1] of sub-queue 0 counts the finished workgroups.
+// prefix sum).
 // One round of vector loads over the scene record's 64-byte lines, a lane
 // each, before a wave's first ray: a wave of this pass runs nearly alone on
 // its CU after the march has filled L2 with framebuffer lines, so the scalar
@@ -145,7 +144,6 @@ template <bool ESCAPE, bool SPH>
 __device__ __forceinline__ void band_rays(const DevScene& s, const DevOut& out, const DevQueue& q,
                                           uint32_t blk, uint32_t R, uint32_t nband) {
   __shared__ uint32_t pre[kQueueSubs + 1];
-  __shared__ uint32_t last;
   const uint32_t lane = threadIdx.x;
   if (blk < kQueueSubs * R) {
     const uint32_t k = blk % kQueueSubs, part = blk / kQueueSubs;
@@ -187,19 +185,6 @@ __device__ __forceinline__ void band_rays(const DevScene& s, const DevOut& out, 
                             (int)(idx / (uint32_t)s.W), 0u);
     }
   }
-  // Every lane's reads of the counts have returned before the barrier, so
-  // the reset cannot race with them; the queue is read again only by later
-  // launches.  (No device-scope fence here: on this multi-XCD part it writes
-  // back and invalidates the XCD's L2, full of framebuffer lines, in every
-  // workgroup.)
-  __syncthreads();
-  if (lane == 0) last = atomicAdd(q.count + 1, 1u) == kQueueSubs * R + nband - 1u ? 1u : 0u;
-  __syncthreads();
-  if (last) {
-    atomicExch(q.count + 16 * lane, 0u);
-    atomicExch(q.count + 16 * lane + 2, 0u);
-    if (lane == 0) atomicExch(q.count + 1, 0u);
-  }
 }
 
 // Workgroups of the FP64 pass of one frame: edge workgroups per sub-queue and
@@ -229,6 +214,17 @@ __global__ __launch_bounds__(64) void band_frames_kernel(const DevScene* __restr
 __global__ void zero_u32_kernel(uint32_t* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
+}
+
+// Scene record and queue counts of a frame in place.  A kernel rather than
+// hipMemcpyAsync / hipMemsetAsync, so the call may also be captured in a
+// graph.
+__global__ __launch_bounds__(256) void scene_kernel(DevScene s, DevScene* dst, uint32_t* count) {
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
+  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+  for (uint32_t i = threadIdx.x; i < sizeof(DevScene) / 4; i += 256) d[i] = src[i];
+  if (count)
+    for (uint32_t i = threadIdx.x; i < kQueueCountWords; i += 256) count[i] = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -295,8 +291,7 @@ hipError_t launch_turning(const DevScene* scene, double* l, int W, int H, hipStr
   return hipGetLastError();
 }
 
-// FP64 pass of one frame; the last workgroup clears the queue, so it is clear
-// when the launch completes.
+// FP64 pass of one frame.
 hipError_t launch_band(const DevScene* scene, const DevOut& out, const DevQueue& q,
                        hipStream_t stream, bool escape, bool spheres) {
   const dim3 g(kEdgeParts1 * kQueueSubs + kBandWaves1), b(64);
@@ -379,6 +374,14 @@ hipError_t launch_band_frames(const DevScene* scenes, const DevOut& out, int W, 
 
 hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t stream) {
   hipLaunchKernelGGL(zero_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, p, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_scene(const DevScene& s, DevScene* dst, uint32_t* count, hipStream_t stream) {
+  static_assert(sizeof(DevScene) % 4 == 0, "scene record is copied as 32-bit words");
+  static_assert(sizeof(DevScene) + 2 * sizeof(void*) <= 4096,
+                "the scene record is passed as a kernel argument");
+  hipLaunchKernelGGL(scene_kernel, dim3(1), dim3(256), 0, stream, s, dst, count);
   return hipGetLastError();
 }
 

@@ -17,18 +17,6 @@ constexpr size_t kScratchBytes = kSceneBytes + kCountBytes + kNoallocQueueItems 
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// Copy the scene record into the array and clear the queue's counts (the
-// array keeps the previous call's contents).  A kernel rather than
-// hipMemcpyAsync / hipMemsetAsync, so the call may also be captured in a
-// graph.
-__global__ __launch_bounds__(256) void noalloc_setup_kernel(DevScene s, DevScene* dst,
-                                                            uint32_t* count) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
-  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-  for (uint32_t i = threadIdx.x; i < sizeof(DevScene) / 4; i += blockDim.x) d[i] = src[i];
-  for (uint32_t i = threadIdx.x; i < kQueueCountWords; i += blockDim.x) count[i] = 0u;
-}
-
 }  // namespace
 
 hipError_t noalloc_scratch(void** ptr) {
@@ -42,14 +30,6 @@ NoallocLayout noalloc_layout(void* base) {
   l.count = reinterpret_cast<uint32_t*>(b + kSceneBytes);
   l.items = reinterpret_cast<uint64_t*>(b + kSceneBytes + kCountBytes);
   return l;
-}
-
-hipError_t launch_noalloc_setup(const DevScene& s, const NoallocLayout& l, hipStream_t stream) {
-  static_assert(sizeof(DevScene) % 4 == 0, "scene record is copied as 32-bit words");
-  static_assert(sizeof(DevScene) + 2 * sizeof(void*) <= 4096,
-                "the scene record is passed as a kernel argument");
-  hipLaunchKernelGGL(noalloc_setup_kernel, dim3(1), dim3(256), 0, stream, s, l.scene, l.count);
-  return hipGetLastError();
 }
 
 }  // namespace bh
