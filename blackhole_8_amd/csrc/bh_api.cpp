@@ -199,6 +199,7 @@ int build_scene(bh_ctx* ctx, const bh_scene* sc, const bh_options* opt_in, DevSc
   d->M = sc->hole.mass;
   d->bc = 3.0 * std::sqrt(3.0) * d->M;  // b_c (blackhole_solution.h:25)
   d->Rh = 2 * d->M;                     // radius() (blackhole_solution.h:57)
+  d->Rcull = d->Rh * (1.0 + 1e-6);
   d->l0 = std::cbrt(DBL_EPSILON);       // epsilon<double>() (utility.h:17-21)
   const double r0 = std::sqrt(d->F[0] * d->F[0] + d->F[1] * d->F[1] + d->F[2] * d->F[2]);
   if (!(r0 > 0.0)) return fail(ctx, BH_ERR_INVALID_ARG, "camera coincides with the hole");

@@ -1,4 +1,4 @@
-// bh_fp64.h — the reference march in FP64, one lane per ray, in the
+// bh_fp64.h — the parts of the reference march in FP64, one lane per ray, in the
 // reference's operation order (the library is compiled with
 // -ffp-contract=off, so every product and sum rounds once, as written).
 //
@@ -74,7 +74,7 @@ __device__ inline double solve_g64(double b, double M, double l0, int root) {
 // Orbit-plane frame of one pixel (blackhole_solution_test.cc:167-183).
 struct Frame64 {
   double R[9];  // [zv yv xv] as columns
-  double b, r0, phi0, u0, u_end, du, du_h;
+  double b, X0, Y0, r0, phi0, u0, u_end, du, du_h;  // (X0, Y0, b): R^-1 F
   bool captured, degenerate;
 };
 
@@ -151,6 +151,8 @@ __device__ inline void frame64(const DevScene& s, int x, int y, Frame64& f) {
   f.captured = sol < 0;
   f.u_end = b < s.bc ? 1.0 / (3 * M) : sol;
   f.b = b;
+  f.X0 = Fp.x;
+  f.Y0 = Fp.y;
   f.r0 = sqrt(dot(Fp, Fp));
   f.phi0 = atan(Fp.z / Fp.y);
   f.u0 = 1. / f.r0;
@@ -204,7 +206,7 @@ struct Hit64 {
 
 // (sphere i is tested when bit i of smask is set; the hole and the disc always)
 __device__ inline bool find_collision64(const DevScene& s, d3 p1, d3 p2, Hit64* h,
-                                        uint32_t smask = ~0u) {
+                                        uint32_t smask) {
   bool found = false;
   double best = 0;
   d3 q;
@@ -299,8 +301,10 @@ __device__ inline uint32_t disc_color64(const DevScene& s, d3 p) {
   double r = sqrt(dot(v, v));
   double theta = acos(dot(s1, v) / (sqrt(dot(s1, s1)) * r));
   theta = isnan(theta) ? 0 : theta;
-  double a = (r * cos(theta) / sqrt(dot(s1, s1))) * t.cols;
-  double b = (r * sin(theta) / sqrt(dot(s2, s2))) * t.rows;
+  double sn, cs;
+  sincos(theta, &sn, &cs);  // the values of sin and cos, from one reduction
+  double a = (r * cs / sqrt(dot(s1, s1))) * t.cols;
+  double b = (r * sn / sqrt(dot(s2, s2))) * t.rows;
   if (s.filter == BH_FILTER_BILINEAR) return bilinear64(t, a, b);
   return texel(t, tex_index(a, t.cols), tex_index(b, t.rows));
 }
@@ -337,179 +341,6 @@ struct Pixel64 {
   d3 q;
   int steps;
 };
-
-// The spheres (a bit each) that a chord of the march in frame f can meet.
-// Every point of the march is B + yv r cos(phi) + xv r sin(phi) (matrow with
-// the first component 0) or the camera or B, all in the plane through B
-// spanned by yv and xv (R's second and third columns) up to rounding of
-// ~1e-15 (r + |B|), with r <= reach when du > 0 (u only grows from u0, or
-// the escape march stops short of r_esc).  A sphere whose centre lies farther
-// from that plane than R + tol misses every chord in exact arithmetic by
-// D^2 - R^2 >= 1e-12 L^2, L bounding |q - c| over the march's points q, far
-// above the rounding of seg_sphere64's discriminant (~1e-15 |Q|^2 L^2 against
-// its exact |Q|^2 (R^2 - D^2)), so its test would return false on every
-// chord: skipping it changes no outcome.  With du <= 0 (or not finite) the
-// points are not bounded and every sphere is kept.
-__device__ inline uint32_t plane_spheres64(const DevScene& s, const Frame64& f) {
-  if (!(f.du > 0.0) || !(f.r0 < 1e300)) return ~0u;
-  const d3 yv = mk3(f.R[1], f.R[4], f.R[7]), xv = mk3(f.R[2], f.R[5], f.R[8]);
-  const d3 n = normalize(cross(yv, xv));
-  if (!(dot(n, n) > 0.5)) return ~0u;
-  const d3 B = ld3(s.B);
-  const double reach = s.escape ? fmax(f.r0, s.r_esc) : f.r0;
-  const double bs = sqrt(dot(B, B));
-  uint32_t m = 0u;
-  for (int i = 0; i < s.n_spheres; ++i) {
-    const d3 c = ld3(s.sc[i]) - B;
-    const double R = s.sr[i];
-    const double tol = 1e-6 * (sqrt(dot(c, c)) + reach + R) + 1e-9 * bs;
-    if (!(fabs(dot(n, c)) > R + tol)) m |= 1u << i;
-  }
-  return m;
-}
-
-// The whole march of one pixel (blackhole_solution_test.cc:167-298) with the
-// escape extension.  Returns through px.
-__device__ inline void trace64(const DevScene& s, int x, int y, Pixel64& px) {
-  Frame64 f;
-  frame64(s, x, y, f);
-  const double nan = __builtin_nan("");
-  px.q = mk3(nan, nan, nan);
-  if (f.degenerate) {
-    px.rgb = 0;
-    px.cls = BH_HIT_HORIZON;
-    px.phi = nan;
-    px.steps = 0;
-    return;
-  }
-  const d3 B = ld3(s.B);
-  const double M = s.M;
-  double u = f.u0, w_prev = 0, phi = f.phi0;
-  d3 P_prev = ld3(s.C), P_prev2 = P_prev;
-  int steps = 0;
-  Hit64 h;
-  bool hit = false;
-  const int nstep = s.nstep;
-  const uint32_t smask = plane_spheres64(s, f);
-
-  // One step at the current u (the caller advances u).
-  auto step = [&]() -> bool {
-    double w = 1.0 / sqrt(G64(u, f.b, M));
-    phi += (w_prev + w) * f.du_h;
-    double r = 1. / u;
-    d3 lv = mk3(0, r * cos(phi), r * sin(phi));
-    d3 P = matrow(f.R, lv) + B;
-    w_prev = w;
-    ++steps;
-    if (find_collision64(s, P_prev, P, &h, smask)) return true;
-    P_prev2 = P_prev;
-    P_prev = P;
-    return false;
-  };
-
-  for (int i = 0; i < nstep - 1 && !hit; ++i) {
-    u += f.du;
-    hit = step();
-  }
-  if (!hit) {
-    u += f.du * 0.9;
-    hit = step();
-  }
-  if (!hit && f.captured) {
-    if (find_collision64(s, P_prev, B, &h, smask)) {
-      hit = true;
-    } else {
-      px.rgb = 0;
-      px.cls = BH_HIT_NONE;
-      px.phi = phi;
-      px.steps = steps;
-      return;
-    }
-  }
-  if (!hit) {
-    for (int i = 0; i < nstep - 1 && !hit; ++i) {
-      u -= f.du;
-      hit = step();
-    }
-  }
-  if (!hit && s.escape) {
-    while (steps < s.step_cap && !hit) {
-      double un = u - f.du;
-      if (un * s.r_esc <= 1.0) break;
-      u = un;
-      hit = step();
-    }
-  }
-  if (hit) {
-    px.rgb = hit_color64(s, h);
-    px.cls = h.cls;
-    px.q = h.q;
-  } else {
-    px.rgb = 0;
-    px.cls = BH_HIT_NONE;
-    if (s.escape && s.has_bg) px.rgb = equirect64(s.bg, normalize(P_prev - P_prev2));
-  }
-  px.phi = phi;
-  px.steps = steps;
-}
-
-// The reference march of pixel (x, y) replayed for a known outcome: the march
-// ends at step n with a disc hit (cls BH_HIT_DISC) or with no hit (escape
-// background along the last chord).  The swept angle of steps 1..n follows
-// trace64's loop to the bit (the same updates of u, w and phi in the same
-// order); only the last chord's two end points are placed, and the colour is
-// taken as trace64 takes it, without the per-step positions and object tests.
-// Returns false when the last chord does not cross the disc after all (the
-// outcome was not the reference's); px is then unset.
-__device__ inline bool replay64(const DevScene& s, int x, int y, int n, int cls, Pixel64& px) {
-  Frame64 f;
-  frame64(s, x, y, f);
-  if (f.degenerate || n < 1) return false;
-  const d3 B = ld3(s.B);
-  const double M = s.M;
-  const int nstep = s.nstep;
-  double u = f.u0, w_prev = 0, phi = f.phi0;
-  double u_a = u, phi_a = phi;  // state at the start of the last chord
-  for (int k = 1; k <= n; ++k) {
-    u_a = u;
-    phi_a = phi;
-    if (k < nstep)
-      u += f.du;
-    else if (k == nstep)
-      u += f.du * 0.9;
-    else
-      u -= f.du;
-    double w = 1.0 / sqrt(G64(u, f.b, M));
-    phi += (w_prev + w) * f.du_h;
-    w_prev = w;
-  }
-  auto place = [&](double uu, double ph) {
-    double r = 1. / uu;
-    d3 lv = mk3(0, r * cos(ph), r * sin(ph));
-    return matrow(f.R, lv) + B;
-  };
-  const d3 Pb = place(u, phi);
-  const d3 Pa = n == 1 ? ld3(s.C) : place(u_a, phi_a);
-  const double nan = __builtin_nan("");
-  px.phi = phi;
-  px.steps = n;
-  if (cls == BH_HIT_DISC) {
-    Hit64 h;
-    h.cls = BH_HIT_DISC;
-    h.index = -1;
-    if (!s.has_disc || !annulus64(s, Pa, Pb, &h.q)) return false;
-    px.rgb = hit_color64(s, h);
-    px.cls = BH_HIT_DISC;
-    px.q = h.q;
-    return true;
-  }
-  if (cls != BH_HIT_NONE) return false;
-  px.rgb = 0;
-  px.cls = BH_HIT_NONE;
-  px.q = mk3(nan, nan, nan);
-  if (s.escape && s.has_bg) px.rgb = equirect64(s.bg, normalize(Pb - Pa));
-  return true;
-}
 
 __device__ inline void store_pixel64(const DevOut& o, size_t idx, const Pixel64& p) {
   if (o.rgb) {

@@ -28,6 +28,7 @@ struct DevScene {
   double B[3];
   double F[3];     // C - B
   double M, bc, Rh;
+  double Rcull;    // Rh (1 + 1e-6): a chord that stays farther out misses the horizon
   double l0;       // SolveG lower bracket cbrt(DBL_EPSILON) (utility.h:17-21)
   double u0;       // 1 / |C - B|
   // disc (Annulus)

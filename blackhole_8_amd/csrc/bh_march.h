@@ -7,7 +7,7 @@
 
 #include <type_traits>
 
-#include "bh_math.h"
+#include "bh_trace64.h"
 
 namespace bh {
 

@@ -19,8 +19,8 @@ namespace bh {
 // ---------------------------------------------------------------------------
 // FP64 reference march
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void march64_kernel(const DevScene* __restrict__ sp,
-                                                      DevOut out) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void march64_kernel(const DevScene* __restrict__ sp, DevOut out) {
   const DevScene& s = *sp;
   const int x = blockIdx.x * 16 + (threadIdx.x & 15);
   const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
