@@ -195,20 +195,63 @@ template <> __device__ __forceinline__ void sincos_swept<double>(double a, doubl
 
 constexpr float kTwoPiF = 6.28318531f;
 
-// Spheres (the slots of L).  A sphere of radius R whose centre lies at
-// distance z from the plane cuts it in a circle of radius sqrt(R^2 - z^2), and
+// Moves the window of slot k on to the ray's next revolution when it ends
+// before swept angle ab.
+template <typename T>
+__device__ __forceinline__ void next_window(Lane<T>& L, int k, float ab) {
+  const float hi = L.slo[k] + L.sw[k];
+  if (ab > hi) L.slo[k] += kTwoPiF * (__builtin_floorf((ab - hi) * (1.f / kTwoPiF)) + 1.f);
+}
+
+// FP64 lanes: the sphere slots (a bit each) that the step chord from kappa = ka
+// to kb, ending at swept angle ab after an increment d, can meet (every slot
+// when all), with the windows that end before ab moved on.  A slot's window
+// must meet the chord's wedge and its circle the chord's radii: every point of
+// the chord lies no farther from B than its farther end and no nearer than
+// cos(d/2) >= 1 - d^2/8 of its nearer end, here with a margin of 1e-3 of the
+// circle's distance, far above the FP32 errors.  Most chords in a window lie
+// off its circle's radii (720p frame with 16 spheres: FP64 pass 66 us when
+// every one was tested, 39 us this way).  FP32 lanes test every chord in a
+// window: there the check costs as much as it saves.
+__device__ __forceinline__ uint32_t sphere_mask(const DevScene& s, Lane<double>& L, double ka,
+                                                double kb, float ab, float d, bool all) {
+  const float ra = __builtin_amdgcn_rcpf((float)__builtin_fma(ka, L.du, L.u0));
+  const float rb = __builtin_amdgcn_rcpf((float)__builtin_fma(kb, L.du, L.u0));
+  const float rmax = fmaxf(ra, rb) * 1.001f;
+  const float rmin = fminf(ra, rb) * __builtin_fmaf(-0.125f * d, d, 1.f) * 0.999f;
+  uint32_t mask = 0u;
+  double nxt = 1e308;
+#pragma unroll
+  for (int k = 0; k < kSphSlots<double>; ++k) {
+    if (k >= L.ns) continue;
+    if (all || ab >= L.slo[k]) {
+      const float X = (float)L.sx[k], Y = (float)L.sy[k];
+      const float dc = __builtin_amdgcn_sqrtf(X * X + Y * Y);
+      const float rho = __builtin_amdgcn_sqrtf(fmaxf((float)L.srho2[k], 0.f));
+      const float m = 1e-3f * (dc + rho);
+      if (all || !(rmax < dc - rho - m || rmin > dc + rho + m)) mask |= 1u << k;
+    }
+    next_window(L, k, ab);
+    nxt = fmin(nxt, (double)L.slo[k]);
+  }
+  L.a_sph = nxt;
+  return mask;
+}
+
+// A sphere of radius R whose centre lies at distance z from the plane cuts it in a circle of radius sqrt(R^2 - z^2), and
 // |P - c|^2 = |P - c'|^2 + z^2 for a point P of the plane and the centre's
 // projection c', so the reference's segment/sphere test
 // (blackhole_solution.h:65-88, the same test as the horizon's) of an in-plane
 // chord is exactly this circle test in the plane.  The chord from
 // P_a = (ra, 0) to P_b = (bx, by), in the frame rotated by the swept angle aa
-// (sa, ca its sine and cosine), is tested against the slots whose window its
-// wedge meets (every slot when all); a hit nearer to the chord start than
-// best (found) replaces hit.  ab is the swept angle at the chord's end: a
-// window that ends before it moves on to the ray's next revolution.
+// (sa, ca its sine and cosine), is tested against the slots in mask (FP64) or
+// those whose window its wedge meets, every slot when all (FP32, whose windows
+// that end before ab, the chord's end, then move on); a hit nearer to the
+// chord start than best (found) replaces hit.
 template <typename T>
 __device__ inline bool sphere_slots(const DevScene& s, Lane<T>& L, T ra, T sa, T ca, double aa,
-                                    T bx, T by, float ab, bool all, bool found, T best,
+                                    T bx, T by, float ab, bool all, uint32_t mask,
+                                    bool found, T best,
                                     HitRec<T>& hit) {
   const T qx = bx - ra, qy = by;
   const T qq = qx * qx + qy * qy;
@@ -217,7 +260,7 @@ __device__ inline bool sphere_slots(const DevScene& s, Lane<T>& L, T ra, T sa, T
 #pragma unroll
   for (int k = 0; k < kSphSlots<T>; ++k) {
     if (k >= L.ns) continue;
-    if (all || ab >= L.slo[k]) {
+    if (sizeof(T) == 8 ? ((mask >> k) & 1u) != 0u : (all || ab >= L.slo[k])) {
       const T X = L.sx[k], Y = L.sy[k], rho2 = L.srho2[k];
       // centre in the rotated frame, then P_a - c' and P_b - c'
       const T xc = X * ca + Y * sa, yc = Y * ca - X * sa;
@@ -253,42 +296,45 @@ __device__ inline bool sphere_slots(const DevScene& s, Lane<T>& L, T ra, T sa, T
         }
       }
     }
-    const float hi = L.slo[k] + L.sw[k];
-    if (ab > hi) L.slo[k] += kTwoPiF * (__builtin_floorf((ab - hi) * (1.f / kTwoPiF)) + 1.f);
-    nxt = fmin(nxt, (double)L.slo[k]);
+    if constexpr (sizeof(T) == 4) {
+      next_window(L, k, ab);
+      nxt = fmin(nxt, (double)L.slo[k]);
+    }
   }
-  L.a_sph = nxt;
+  if constexpr (sizeof(T) == 4) L.a_sph = nxt;
   return found;
 }
 
-// The step chord from (ka, aa) to (kb, aa + da) against the spheres; ab and
-// all as for sphere_slots.
+// The step chord from (ka, aa) to (kb, aa + da) against the spheres; ab, all
+// and mask as for sphere_slots.
 template <typename T>
 __device__ inline bool sphere_chord(const DevScene& s, Lane<T>& L, T ka, double aa, T kb, T da,
-                                    float ab, bool all, bool found, T best, HitRec<T>& hit) {
+                                    float ab, bool all, uint32_t mask, bool found, T best,
+                                    HitRec<T>& hit) {
   const T ra = rcp<T>(fma_t<T>(ka, L.du, L.u0));
   const T rb = rcp<T>(fma_t<T>(kb, L.du, L.u0));
   T sd, cd, sa, ca;
   sincos_t<T>(da, &sd, &cd);
   sincos_swept<T>(aa, &sa, &ca);
-  return sphere_slots<T>(s, L, ra, sa, ca, aa, rb * cd, rb * sd, ab, all, found, best, hit);
+  return sphere_slots<T>(s, L, ra, sa, ca, aa, rb * cd, rb * sd, ab, all, mask, found, best, hit);
 }
 
 // A captured ray's last chord, from its last point (kappa = nstep - 0.1, at
 // the swept angle a) straight to B (blackhole_solution_test.cc:264-272): it
 // enters the horizon at distance r - R_h, unless a sphere is met before.
-template <typename T>
+template <typename T, bool SPH>
 __device__ inline void captured_chord(const DevScene& s, Lane<T>& L, double a, HitRec<T>& hit) {
   hit.cls = BH_HIT_HORIZON;
   hit.ang = a;
   hit.hx = (T)s.Rh;
   hit.hy = (T)0;
+  if constexpr (!SPH) return;
   if (L.ns > 0) {
     const T ra = rcp<T>(fma_t<T>((T)s.nstep - (T)0.1, L.du, L.u0));
     const T dh = ra - (T)s.Rh;
     T sa, ca;
     sincos_swept<T>(a, &sa, &ca);
-    sphere_slots<T>(s, L, ra, sa, ca, a, (T)0, (T)0, (float)a, true, true, dh * dh, hit);
+    sphere_slots<T>(s, L, ra, sa, ca, a, (T)0, (T)0, (float)a, true, ~0u, true, dh * dh, hit);
   }
 }
 
@@ -390,12 +436,13 @@ __device__ __forceinline__ void advance(const Lane<T>& L, MarchState<T>& st, T G
 // The exact chord tests of the step just advanced (from angle a_prev to st.a,
 // increment st.d), if it is an event (a crossing angle passed, the horizon
 // guard exceeded, or force).  Returns true when the chord hits (hit is
-// filled).  With SPH the chord is also tested against the spheres whose
-// window it meets.
+// filled).  With SPH the chord is also tested against the spheres whose window
+// it meets (FP64: those in mask), every slot on a chord of Da >= 1 (the wedge
+// argument needs Da < pi; phi_safe < pi on an armed lane, +inf on an ended one).
 template <typename T, typename S, bool SPH = false>
 __device__ __forceinline__ bool step_tests(const S& s, Lane<T>& L, const MarchState<T>& st,
                                            double a_prev, double first_aa, T ka, T kb,
-                                           bool force, HitRec<T>& hit) {
+                                           bool force, HitRec<T>& hit, uint32_t mask = 0u) {
   const bool eh = (float)st.d > L.phi_safe;
   const double aa = force ? first_aa : a_prev;
   const T da = force ? (T)(st.a - first_aa) : st.d;
@@ -407,11 +454,9 @@ __device__ __forceinline__ bool step_tests(const S& s, Lane<T>& L, const MarchSt
     if (!found && st.a >= L.a_ev) L.a_ev = next_event(st.a, chi0_of(L), L.guard);
   }
   if constexpr (SPH) {
-    // every slot on a chord of Da >= 1 (the wedge argument needs Da < pi;
-    // phi_safe < pi on an armed lane, +inf on an ended one)
     const bool all = force || (float)st.d > fmaxf(1.f, L.phi_safe);
-    if (all || st.a >= L.a_sph)
-      found = sphere_chord<T>(s, L, ka, aa, kb, da, (float)st.a, all, found, best, hit);
+    if (sizeof(T) == 8 ? mask != 0u : (all || st.a >= L.a_sph))
+      found = sphere_chord<T>(s, L, ka, aa, kb, da, (float)st.a, all, mask, found, best, hit);
   }
   return found;
 }
@@ -425,7 +470,7 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
   return step_tests<T, S, SPH>(s, L, st, st.a - (double)st.d, first_aa, ka, kb, force, hit);
 }
 
-// The march of one ray in precision T.  first_aa is the angle of the camera
+// The march of one FP32 ray.  first_aa is the angle of the camera
 // in the (e1, e2) frame: 0 when Y0 > 0, pi when Y0 < 0 (the reference's
 // phi0 = atan(b/Y0) then points away from the camera, and only the first
 // chord starts at the camera itself).
@@ -453,7 +498,8 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
   // without sphere slots (fewer checks and single tail steps: 20 steps leave
   // none inbound and one outbound; nine-step blocks measured no faster and
   // spill), four otherwise (six would cost the sphere lanes occupancy)
-  constexpr int kB = (NS > 0 && sizeof(T) == 4 && !SPH) ? 6 : 4;
+  static_assert(sizeof(T) == 4, "FP64 lanes take march64e");
+  constexpr int kB = (NS > 0 && !SPH) ? 6 : 4;
   MarchState<T> st{(T)0, 0.0, (T)0};
   o.hit.cls = BH_HIT_NONE;
   o.hit.obj = 0;
@@ -506,83 +552,50 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
   // FP64 additions.  The replay forms its intermediate angles as a0
   // plus the FP32 partial sums of the increments (monotone, below the
   // block's sum by at least the last increment) and ends on the block's own
-  // angle; each chord starts where the previous one ended.  FP64 lanes sum
-  // every increment in FP64.
+  // angle; each chord starts where the previous one ended.
   auto block = [&](int n0, auto coeffs, bool inbound, auto len) {
     constexpr int K = decltype(len)::value;
     const double a0 = st.a;
-    if constexpr (sizeof(T) == 4) {
-      const T w0 = st.w;
-      T wk[K];
+    const T w0 = st.w;
+    T wk[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      T G, ka, kb;
+      coeffs(n0 + k, &G, &ka, &kb);
+      wk[k] = rsq<T>(G);
+    }
+    T mid = wk[0];
+#pragma unroll
+    for (int k = 1; k < K - 1; ++k) mid += wk[k];
+    const T sum = __builtin_fmaf(2.f, mid, w0 + wk[K - 1]);
+    st.w = wk[K - 1];
+    st.a = a0 + (double)sum;
+    const T dlast = wk[K - 2] + wk[K - 1];
+    // the last increment is read after the block only by end_ray, which
+    // an outbound block's successor may call before stepping
+    if (inbound || n0 + 2 * K > 2 * nstep) st.d = dlast;
+    const float dmax = inbound ? dlast : w0 + wk[0];
+    bool ev = dmax > L.phi_safe || st.a >= L.a_ev;
+    if constexpr (SPH) ev = ev || dmax > fmaxf(1.f, L.phi_safe) || st.a >= L.a_sph;
+    if (ev) {
+      // the block's angles are recomputed from a0 rather than kept (more
+      // live VGPRs in the fast path would cost occupancy): an empty asm
+      // statement hides from the compiler that the copy equals a0
+      double ar = a0;
+      __asm__ volatile("" : "+v"(ar));
+      const double a_end = st.a;
+      double ap = ar;
+      T part = (T)0;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         T G, ka, kb;
         coeffs(n0 + k, &G, &ka, &kb);
-        wk[k] = rsq<T>(G);
-      }
-      T mid = wk[0];
-#pragma unroll
-      for (int k = 1; k < K - 1; ++k) mid += wk[k];
-      const T sum = __builtin_fmaf(2.f, mid, w0 + wk[K - 1]);
-      st.w = wk[K - 1];
-      st.a = a0 + (double)sum;
-      const T dlast = wk[K - 2] + wk[K - 1];
-      // the last increment is read after the block only by end_ray, which
-      // an outbound block's successor may call before stepping
-      if (inbound || n0 + 2 * K > 2 * nstep) st.d = dlast;
-      const float dmax = inbound ? dlast : w0 + wk[0];
-      bool ev = dmax > L.phi_safe || st.a >= L.a_ev;
-      if constexpr (SPH) ev = ev || dmax > fmaxf(1.f, L.phi_safe) || st.a >= L.a_sph;
-      if (ev) {
-        // the block's angles are recomputed from a0 rather than kept (more
-        // live VGPRs in the fast path would cost occupancy): an empty asm
-        // statement hides from the compiler that the copy equals a0
-        double ar = a0;
-        __asm__ volatile("" : "+v"(ar));
-        const double a_end = st.a;
-        double ap = ar;
-        T part = (T)0;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          T G, ka, kb;
-          coeffs(n0 + k, &G, &ka, &kb);
-          st.d = (k == 0 ? w0 : wk[k - 1]) + wk[k];
-          part = k == 0 ? st.d : part + st.d;
-          st.a = k == K - 1 ? a_end : ar + (double)part;
-          if (step_tests<T, DevScene, SPH>(s, L, st, ap, first_aa, ka, kb, false, o.hit))
-            end_ray(n0 + k);
-          ap = st.a;
-        }
-      }
-    } else {
-      static_assert(K == 4, "FP64 lanes march four-step blocks");
-      T dk[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        T G, ka, kb;
-        coeffs(n0 + k, &G, &ka, &kb);
-        advance<T>(L, st, G);
-        dk[k] = st.d;
-      }
-      const float dmax = (float)(inbound ? dk[3] : dk[0]);
-      bool ev = dmax > L.phi_safe || st.a >= L.a_ev;
-      if constexpr (SPH) ev = ev || dmax > fmaxf(1.f, L.phi_safe) || st.a >= L.a_sph;
-      if (ev) {
-        // the replay recomputes the four sums from a0 (the same FP64
-        // additions) rather than keeping them live
-        double ar = a0;
-        __asm__ volatile("" : "+v"(ar));
-        st.a = ar;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          T G, ka, kb;
-          coeffs(n0 + k, &G, &ka, &kb);
-          st.d = dk[k];
-          st.a += (double)dk[k];
-          if (step_tests<T, DevScene, SPH>(s, L, st, st.a - (double)st.d, first_aa, ka, kb,
-                                           false, o.hit))
-            end_ray(n0 + k);
-        }
+        st.d = (k == 0 ? w0 : wk[k - 1]) + wk[k];
+        part = k == 0 ? st.d : part + st.d;
+        st.a = k == K - 1 ? a_end : ar + (double)part;
+        if (step_tests<T, DevScene, SPH>(s, L, st, ap, first_aa, ka, kb, false, o.hit))
+          end_ray(n0 + k);
+        ap = st.a;
       }
     }
   };
@@ -616,14 +629,7 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
     // captured: chord to the centre; the horizon is always entered
     // (r > 3M > 2M) and the disc test sees n.(B - B) = 0 (:264-272)
     if (captured && armed()) {
-      if constexpr (SPH) {
-        captured_chord<T>(s, L, st.a, o.hit);
-      } else {
-        o.hit.cls = BH_HIT_HORIZON;
-        o.hit.ang = st.a;
-        o.hit.hx = (T)s.Rh;
-        o.hit.hy = (T)0;
-      }
+      captured_chord<T, SPH>(s, L, st.a, o.hit);
       end_ray(nstep);
     }
     if (!__any(armed())) goto done;
@@ -804,26 +810,22 @@ __device__ inline bool setup_spheres(const DevScene& s, const T e1[3], const T e
   L.a_sph = 1e308;
   L.sredo = false;
   bool ok = true;
-  for (int i = 0; i < s.n_spheres; ++i) {
-    T c0, c1, c2, R;
+  // a sphere's centre relative to B and its radius
+  auto sphere = [&](int i, T* c0, T* c1, T* c2, T* R) {
     if constexpr (sizeof(T) == 4) {
-      c0 = s.sphf[i][0];
-      c1 = s.sphf[i][1];
-      c2 = s.sphf[i][2];
-      R = s.sphf[i][3];
+      *c0 = s.sphf[i][0];
+      *c1 = s.sphf[i][1];
+      *c2 = s.sphf[i][2];
+      *R = s.sphf[i][3];
     } else {
-      c0 = s.sc[i][0] - s.B[0];
-      c1 = s.sc[i][1] - s.B[1];
-      c2 = s.sc[i][2] - s.B[2];
-      R = s.sr[i];
+      *c0 = s.sc[i][0] - s.B[0];
+      *c1 = s.sc[i][1] - s.B[1];
+      *c2 = s.sc[i][2] - s.B[2];
+      *R = s.sr[i];
     }
-    const T Z = c0 * n0 + c1 * n1 + c2 * n2;
-    const T Rm = R * margin;
-    if (!(Z * Z < Rm * Rm)) continue;
-    if (L.ns == kSphSlots<T>) {
-      ok = false;
-      continue;
-    }
+  };
+  // the circle of a sphere that cuts the plane into slot k
+  auto fill = [&](int k, T c0, T c1, T c2, T R, T Z) {
     const T X = c0 * e1[0] + c1 * e1[1] + c2 * e1[2];
     const T Y = c0 * e2[0] + c1 * e2[1] + c2 * e2[2];
     const T rho2 = R * R - Z * Z;
@@ -837,18 +839,42 @@ __device__ inline bool setup_spheres(const DevScene& s, const T e1[3], const T e
       if (lo + w2 < 0.f) lo += kTwoPiF;
     }
 #pragma unroll
-    for (int k = 0; k < kSphSlots<T>; ++k) {
-      if (k == L.ns) {
-        L.sx[k] = X;
-        L.sy[k] = Y;
-        L.srho2[k] = rho2;
-        L.slo[k] = lo;
-        L.sw[k] = w2;
+    for (int j = 0; j < kSphSlots<T>; ++j) {
+      if (j == k) {
+        L.sx[j] = X;
+        L.sy[j] = Y;
+        L.srho2[j] = rho2;
+        L.slo[j] = lo;
+        L.sw[j] = w2;
       }
     }
-    L.sids |= (uint32_t)i << (8 * L.ns);
     L.a_sph = fmin(L.a_sph, (double)lo);
+  };
+  for (int i = 0; i < s.n_spheres; ++i) {
+    T c0, c1, c2, R;
+    sphere(i, &c0, &c1, &c2, &R);
+    const T Z = c0 * n0 + c1 * n1 + c2 * n2;
+    const T Rm = R * margin;
+    if (!(Z * Z < Rm * Rm)) continue;
+    if (L.ns == kSphSlots<T>) {
+      ok = false;
+      continue;
+    }
+    // FP64 lanes form their circles below, slot by slot: a wave of the FP64
+    // pass then forms as many as its fullest lane holds, not as many as its
+    // lanes meet between them (its pass over the 720p frame 39 -> 37 us; in
+    // the FP32 march the loads by lane cost more: 52 -> 61 us)
+    if constexpr (sizeof(T) == 4) fill(L.ns, c0, c1, c2, R, Z);
+    L.sids |= (uint32_t)i << (8 * L.ns);
     ++L.ns;
+  }
+  if constexpr (sizeof(T) == 8) {
+#pragma unroll 1
+    for (int k = 0; k < L.ns; ++k) {
+      T c0, c1, c2, R;
+      sphere((int)((L.sids >> (8 * k)) & 0xffu), &c0, &c1, &c2, &R);
+      fill(k, c0, c1, c2, R, c0 * n0 + c1 * n1 + c2 * n2);
+    }
   }
   if (!ok) L.sredo = true;
   return ok;
@@ -1200,7 +1226,7 @@ __device__ inline bool refine64(const DevScene& s, Lane<double> L, const RaySetu
   if (cls != BH_HIT_DISC && !(ESCAPE && cls == BH_HIT_NONE)) return false;
   double w = 0.0, a = 0.0, a_prev = 0.0, d = 0.0, ka = 0.0, kb = 0.0;
   // the steps in the order of the march, one phase (one step cubic) at a
-  // time; within a phase two steps' G and w are formed together, so that
+  // time; within a phase four steps' G and w are formed together, so that
   // their dependent FP64 chains overlap (the sums keep their order)
   auto add = [&](double wn, double ka_n, double kb_n) {
     d = (w + wn) * L.h;
@@ -1211,19 +1237,16 @@ __device__ inline bool refine64(const DevScene& s, Lane<double> L, const RaySetu
     kb = kb_n;
   };
   auto run = [&](int k0, int k1, auto coeffs) {
-    int k = k0;
-    for (; k + 1 <= k1; k += 2) {
-      double G1, ka1, kb1, G2, ka2, kb2;
-      coeffs(k, &G1, &ka1, &kb1);
-      coeffs(k + 1, &G2, &ka2, &kb2);
-      const double w1 = rsq<double>(G1), w2 = rsq<double>(G2);
-      add(w1, ka1, kb1);
-      add(w2, ka2, kb2);
-    }
-    if (k <= k1) {
-      double G1, ka1, kb1;
-      coeffs(k, &G1, &ka1, &kb1);
-      add(rsq<double>(G1), ka1, kb1);
+#pragma unroll 1
+    for (int k = k0; k <= k1; k += 4) {
+      double G[4], kan[4], kbn[4], wn[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) coeffs(k + i, &G[i], &kan[i], &kbn[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wn[i] = rsq<double>(G[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k + i <= k1) add(wn[i], kan[i], kbn[i]);
     }
   };
   run(1, min(n, nstep - 1), [&](int k, double* G, double* ka_n, double* kb_n) {
@@ -1252,6 +1275,104 @@ __device__ inline bool refine64(const DevScene& s, Lane<double> L, const RaySetu
   double d2;
   return event_chord<double, DevScene>(s, L, ka, aa, kb, a, a - aa, false, true, o.hit, &d2) &&
          o.hit.cls == BH_HIT_DISC;
+}
+
+// The event march of one FP64 ray (march's steps and tests, every increment
+// summed in FP64), for the FP64 pass.  The rays of a wave come from all over
+// the frame, a few per wave and about one wave per SIMD, so what bounds the
+// pass is the length of a wave's dependent work.  Hence, as in trace64, each
+// lane steps on its own, four steps' G and w at a time (their chains overlap),
+// up to its next event, and the lanes' events are tested together: as often as
+// the ray with the most events needs, not once for every step at which some
+// lane has one.
+template <bool ESCAPE, bool SPH>
+__device__ inline void march64e(const DevScene& s, Lane<double>& L, bool captured,
+                                double first_aa, double du64, MarchOut<double>& o) {
+  const int nstep = s.nstep;
+  const double kt = (double)nstep - 0.1;
+  MarchState<double> st{0.0, 0.0, 0.0};
+  o.hit.cls = BH_HIT_NONE;
+  o.hit.obj = 0;
+  o.hit.ang = 0.0;
+  o.hit.hx = o.hit.hy = 0.0;
+  o.du64 = du64;
+  // kappa of the ends of step i's chord
+  auto ends = [&](int i, double* ka, double* kb) {
+    const double ki = (double)i, j = (double)(i - nstep);
+    *kb = i < nstep ? ki : kt - j;
+    *ka = i < nstep ? ki - 1.0 : i == nstep ? kt - 0.9 : kt - j + 1.0;
+  };
+  bool live = true, inbound = true;
+  uint32_t mask = 0u;  // the spheres that the waiting chord can meet
+  double ka, kb;
+  int n = 1;
+#pragma unroll 1
+  do {
+    bool wait = !live;
+#pragma unroll 1
+    do {
+      if (!wait) {
+        // steps n .. n + m - 1 lie in one phase: x = sigma inbound, j after it
+        int last = nstep - 1;
+        double x = (double)(nstep - n), dx = -1.0;
+        if (n >= nstep) {
+          if (inbound) {
+            to_outbound<double>(L);
+            inbound = false;
+          }
+          last = n == nstep ? nstep : n < 2 * nstep ? 2 * nstep - 1 : ESCAPE ? s.step_cap : 0;
+          x = (double)(n - nstep);
+          dx = 1.0;
+        }
+        if (captured && n > nstep) last = 0;
+        if (n > last) live = false;
+        wait = !live;
+        double w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = rsq<double>(step_g<double>(L, x + (double)k * dx));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (n <= last && !wait) {
+            // stop outward before the point would lie at r >= r_escape
+            // (u <= 1 / r_escape)
+            if (ESCAPE && n >= 2 * nstep &&
+                __builtin_fma(kt - (double)(n - nstep), du64, s.u0) * s.r_esc <= 1.0) {
+              wait = true;
+              live = false;
+            } else {
+              st.d = (st.w + w[k]) * L.h;
+              st.w = w[k];
+              st.a += st.d;
+              wait = (float)st.d > L.phi_safe || st.a >= L.a_ev || (n == 1 && first_aa != 0.0);
+              if constexpr (SPH) {
+                const bool all = (float)st.d > fmaxf(1.f, L.phi_safe) ||
+                                 (n == 1 && first_aa != 0.0);
+                mask = 0u;
+                if (all || st.a >= L.a_sph) {
+                  ends(n, &ka, &kb);
+                  mask = sphere_mask(s, L, ka, kb, (float)st.a, (float)st.d, all);
+                }
+                wait = wait || mask != 0u;
+              }
+              if (!wait) ++n;
+            }
+          }
+        }
+      }
+    } while (__any(!wait));
+    if (live) {
+      ends(n, &ka, &kb);
+      live = !step_tests<double, DevScene, SPH>(s, L, st, st.a - st.d, first_aa, ka, kb,
+                                                n == 1 && first_aa != 0.0, o.hit, mask);
+      ++n;  // (a ray that hit ends at the step before n too)
+    }
+  } while (__any(live));
+  o.steps = n - 1;
+  o.a = st.a;
+  o.d = st.d;
+  // captured: chord to the centre; the horizon is always entered
+  // (r > 3M > 2M) and the disc test sees n.(B - B) = 0 (:264-272)
+  if (captured && o.hit.cls == BH_HIT_NONE) captured_chord<double, SPH>(s, L, st.a, o.hit);
 }
 
 // FP64 march of one queued ray: a texel-edge ray's FP32 outcome refined in
@@ -1284,7 +1405,7 @@ __device__ inline void fp64_ray(const DevScene& s, const DevOut& out, size_t idx
       // grazed before the step it names)
       if (SPH || !(outcome != 0u && refine64<ESCAPE>(s, L, r, du, (int)(outcome >> 28),
                                                      (int)(outcome & 0x0fffffffu), mo)))
-        march<double, ESCAPE, SPH>(s, L, r.captured, r.first_aa, du, mo);
+        march64e<ESCAPE, SPH>(s, L, r.captured, r.first_aa, du, mo);
       if (!finish_ray64<ESCAPE>(s, out, idx, e1, e2, r, mo)) return;
       if (replay64(s, x, y, mo.steps, mo.hit.cls, px)) {
         store_pixel64(out, idx, px);

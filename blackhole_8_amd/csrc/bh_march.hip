@@ -145,51 +145,60 @@ __device__ __forceinline__ void band_rays(const DevScene& s, const DevOut& out, 
                                           uint32_t blk, uint32_t R, uint32_t nband) {
   __shared__ uint32_t pre[kQueueSubs + 1];
   const uint32_t lane = threadIdx.x;
-  if (blk < kQueueSubs * R) {
-    const uint32_t k = blk % kQueueSubs, part = blk / kQueueSubs;
-    const uint32_t* count = q.count + 16 * k;
-    const uint64_t* items = q.items + (size_t)k * q.sub_cap;
-    const uint32_t nb = min(count[0], q.sub_cap);
-    const uint32_t ne = min(count[2], q.sub_cap - nb);
-    if (part * 64 < ne) touch_scene(s, lane);
-#pragma unroll 1
-    for (uint32_t i = part * 64 + lane; i < ne; i += R * 64) {
-      const uint64_t it = items[q.sub_cap - 1u - i];
-      const uint32_t idx = (uint32_t)it;
-      fp64_ray<ESCAPE, SPH>(s, out, idx, (int)(idx % (uint32_t)s.W),
-                            (int)(idx / (uint32_t)s.W), (uint32_t)(it >> 32));
-    }
+  // one loop over the rays of either kind, so that both run the same code (an
+  // FP64 ray inlined twice doubles what the instruction cache has to fetch)
+  const bool edge = blk < kQueueSubs * R;
+  uint32_t first, stride, total, k = 0;
+  if (edge) {
+    k = blk % kQueueSubs;
+    const uint32_t nb = min(q.count[16 * k], q.sub_cap);
+    total = min(q.count[16 * k + 2], q.sub_cap - nb);
+    first = blk / kQueueSubs * 64;
+    stride = R * 64;
   } else {
     // pre[k] = band rays of sub-queues 0 .. k-1
-    pre[lane + 1] = min(q.count[16 * lane], q.sub_cap);
-    __syncthreads();
-    if (lane == 0) {
-      pre[0] = 0;
-      for (uint32_t k = 1; k <= kQueueSubs; ++k) pre[k] += pre[k - 1];
+    uint32_t sum = min(q.count[16 * lane], q.sub_cap);
+#pragma unroll
+    for (int j = 1; j < 64; j <<= 1) {
+      const uint32_t v = __shfl_up(sum, j);
+      if (lane >= (uint32_t)j) sum += v;
     }
+    if (lane == 0) pre[0] = 0;
+    pre[lane + 1] = sum;
     __syncthreads();
-    const uint32_t total = pre[kQueueSubs];
-    if ((blk - kQueueSubs * R) * 64 < total) touch_scene(s, lane);
+    total = pre[kQueueSubs];
+    first = (blk - kQueueSubs * R) * 64;
+    stride = nband * 64;
+  }
+  if (first < total) touch_scene(s, lane);
 #pragma unroll 1
-    for (uint32_t j = (blk - kQueueSubs * R) * 64 + lane; j < total; j += nband * 64) {
-      uint32_t lo = 0, hi = kQueueSubs;  // the k with pre[k] <= j < pre[k + 1]
+  for (uint32_t i = first + lane; i < total; i += stride) {
+    uint64_t it;
+    if (edge) {
+      it = q.items[(size_t)k * q.sub_cap + (q.sub_cap - 1u - i)];
+    } else {
+      uint32_t lo = 0, hi = kQueueSubs;  // the lo with pre[lo] <= i < pre[lo + 1]
       while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (pre[mid] <= j)
+        if (pre[mid] <= i)
           lo = mid;
         else
           hi = mid;
       }
-      const uint32_t idx = (uint32_t)q.items[(size_t)lo * q.sub_cap + (j - pre[lo])];
-      fp64_ray<ESCAPE, SPH>(s, out, idx, (int)(idx % (uint32_t)s.W),
-                            (int)(idx / (uint32_t)s.W), 0u);
+      it = (uint32_t)q.items[(size_t)lo * q.sub_cap + (i - pre[lo])];
     }
+    const uint32_t idx = (uint32_t)it;
+    fp64_ray<ESCAPE, SPH>(s, out, idx, (int)(idx % (uint32_t)s.W), (int)(idx / (uint32_t)s.W),
+                          (uint32_t)(it >> 32));
   }
 }
 
 // Workgroups of the FP64 pass of one frame: edge workgroups per sub-queue and
-// band workgroups.
-constexpr uint32_t kEdgeParts1 = 16, kBandWaves1 = 16;     // one frame alone
+// band workgroups (enough that each has at most one wave of rays: an 8K
+// frame's 9,200 band rays in 16 workgroups, nine marches one after another,
+// took 109 us, in 192 it is 22 us; the empty ones cost a small frame nothing
+// measurable).
+constexpr uint32_t kEdgeParts1 = 24, kBandWaves1 = 192;    // one frame alone
 constexpr uint32_t kEdgePartsN = 2, kBandWavesN = 24;      // each frame of a path
 
 template <bool ESCAPE, bool SPH>
