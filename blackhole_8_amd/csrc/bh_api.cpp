@@ -649,6 +649,8 @@ int build_diff(bh_ctx* ctx, const bh_diff_params* p, int precision, bh::DiffScen
     d->az[i] = z.x[i].v;
     d->az_i[i] = z.x[i].t;
   }
+  d->ir0 = 1.0 / std::sqrt(d->C[0] * d->C[0] + d->C[1] * d->C[1] + d->C[2] * d->C[2]);
+  for (int i = 0; i < 3; ++i) d->e1[i] = d->C[i] * d->ir0;
   d->M = p->r_s / 2.0;
   d->bc = 3.0 * std::sqrt(3.0) * d->M;
   d->Rh = 2 * d->M;
@@ -661,7 +663,8 @@ int build_diff(bh_ctx* ctx, const bh_diff_params* p, int precision, bh::DiffScen
   d->vscale = d->tex.rows / (2.0 * p->r_outer);
   d->W = p->width;
   d->H = p->height;
-  d->nstep = 20;
+  d->nstep = bh::kRefSteps;
+  d->inv_nstep = 1.0 / d->nstep;
   return BH_OK;
 }
 

@@ -30,8 +30,8 @@
 //            point, coverage and bilinear texel adjoints give P_bar, hence
 //            (psi_bar, u_bar, e1_bar, e2_bar);
 //   set-up   turning point by implicit differentiation of G(l) = 0, then the
-//            orbit-plane frame in forward mode (tangents: inclination,
-//            distance) contracted with the set-up adjoints.
+//            orbit-plane frame backwards to the pixel point and the camera,
+//            whose tangents along inclination and distance are the scene's.
 // The forward visits a chord's geometry only where something can happen on
 // it: when the orbit angle passes a crossing of the disc plane (closed form
 // per ray) or when a bound on the chord's distance from the centre does not
@@ -51,46 +51,10 @@ constexpr int kThreads = kTile * kTile;
 constexpr int kMaxRec = BH_DIFF_MAX_CROSSINGS;
 constexpr int kPartial = 5;  // r_s, incl, dist, r_in, overflowed rays
 
-// ---------------------------------------------------------------------------
-// Forward-mode FP64 number: value and derivatives along inclination, distance
-// ---------------------------------------------------------------------------
-struct D2 {
-  double v, i, d;
-};
-__device__ __forceinline__ D2 operator+(D2 a, D2 b) { return {a.v + b.v, a.i + b.i, a.d + b.d}; }
-__device__ __forceinline__ D2 operator-(D2 a, D2 b) { return {a.v - b.v, a.i - b.i, a.d - b.d}; }
-__device__ __forceinline__ D2 operator*(D2 a, D2 b) {
-  return {a.v * b.v, a.i * b.v + a.v * b.i, a.d * b.v + a.v * b.d};
+__device__ __forceinline__ double dot3(const double* a, const double* b) {
+  return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
-__device__ __forceinline__ double val(double a) { return a; }
-__device__ __forceinline__ double val(D2 a) { return a.v; }
-__device__ __forceinline__ double rsqrt_n(double a) { return rsq<double>(a); }
-__device__ __forceinline__ D2 rsqrt_n(D2 a) {
-  const double y = rsq<double>(a.v);
-  const double k = -0.5 * y * y * y;
-  return {y, k * a.i, k * a.d};
-}
-__device__ __forceinline__ double sqrt_n(double a) { return sqrt(a); }
-__device__ __forceinline__ D2 sqrt_n(D2 a) {
-  const double y = sqrt(a.v);
-  const double k = 0.5 / y;
-  return {y, k * a.i, k * a.d};
-}
-__device__ __forceinline__ double rcp_n(double a) { return 1.0 / a; }
-__device__ __forceinline__ D2 rcp_n(D2 a) {
-  const double y = 1.0 / a.v;
-  const double k = -y * y;
-  return {y, k * a.i, k * a.d};
-}
-__device__ __forceinline__ void lift(double v, double ti, double td, double& o) { o = v; }
-__device__ __forceinline__ void lift(double v, double ti, double td, D2& o) { o = {v, ti, td}; }
-
-template <typename N> __device__ __forceinline__ N dot3(const N* a, const N* b) {
-  N s = a[0] * b[0];
-  s = s + a[1] * b[1];
-  return s + a[2] * b[2];
-}
-template <typename N> __device__ __forceinline__ void cross3(const N* a, const N* b, N* o) {
+__device__ __forceinline__ void cross3(const double* a, const double* b, double* o) {
   o[0] = a[1] * b[2] - a[2] * b[1];
   o[1] = a[2] * b[0] - a[0] * b[2];
   o[2] = a[0] * b[1] - a[1] * b[0];
@@ -103,45 +67,81 @@ template <typename N> __device__ __forceinline__ void cross3(const N* a, const N
 // b = xv.F, Y0 = yv.F, r0 = |F|.  The reference puts the orbit point at angle
 // phi and radius r at r (cos(phi) yv + sin(phi) xv) starting from
 // phi0 = atan(b / Y0); here the angle psi = phi - phi0 is measured from the
-// camera direction e1 = F / r0 with e2 = (Y0 xv - b yv) / r0, the same point
-// r (cos(psi) e1 + sin(psi) e2) without an arctangent.  (Y0 > 0 for a camera
-// looking at the hole: F.(F - pv) = dist^2 + dist f, so atan(b/Y0) is the
-// polar angle of F and psi = 0 is the camera.)
-template <typename N> struct Frame {
-  N e1[3], e2[3];
-  N b, r0;
+// camera direction e1 = F / r0 with e2 = (Y0 xv - b yv) / r0 = e1 x zv, the
+// same point r (cos(psi) e1 + sin(psi) e2) without an arctangent; and
+// b = zv.(F x yv) = zv.(pv x yv) = |pv x yv|.  (Y0 > 0 for a camera looking at
+// the hole: F.(F - pv) = dist^2 + dist f, so atan(b/Y0) is the polar angle of
+// F and psi = 0 is the camera.)  e1 and r0 are the scene's.
+struct Frame {
+  double e2[3];
+  double b, ib;  // b and 1/b
   bool degenerate;
 };
 
-template <typename N>
-__device__ inline void diff_frame(const DiffScene& s, int px, int py, Frame<N>& f) {
+// The pixel point pv, dv = F - pv and 1/|dv|.
+struct Line {
+  double pv[3], dv[3], ny;
+};
+__device__ __forceinline__ Line pixel_line(const DiffScene& s, int px, int py) {
   const double sx = s.W / 2.0 - px, sy = s.H / 2.0 - py;
-  N pv[3], F[3], dv[3], yv[3], cv[3], zv[3], xv[3];
+  Line l;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    lift(s.fx[k] - s.ay[k] * sx - s.az[k] * sy, s.fx_i[k] - s.ay_i[k] * sx - s.az_i[k] * sy,
-         0.0, pv[k]);
-    lift(s.C[k], s.C_i[k], s.C_d[k], F[k]);
-    dv[k] = F[k] - pv[k];
+    l.pv[k] = s.fx[k] - s.ay[k] * sx - s.az[k] * sy;
+    l.dv[k] = s.C[k] - l.pv[k];
   }
-  const N ny = rsqrt_n(dot3(dv, dv));
+  l.ny = rsq<double>(dot3(l.dv, l.dv));
+  return l;
+}
+
+__device__ inline void diff_frame(const DiffScene& s, int px, int py, Frame& f) {
+  const Line l = pixel_line(s, px, py);
+  double yv[3], cv[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) yv[k] = dv[k] * ny;
-  cross3(pv, yv, cv);
-  const N cc = dot3(cv, cv);
-  f.degenerate = !(val(cc) > 0.0);
-  const N nz = rsqrt_n(f.degenerate ? dot3(dv, dv) : cc);
+  for (int k = 0; k < 3; ++k) yv[k] = l.dv[k] * l.ny;
+  cross3(l.pv, yv, cv);
+  const double cc = dot3(cv, cv);
+  f.degenerate = !(cc > 0.0);
+  f.ib = rsq<double>(f.degenerate ? 1.0 : cc);
+  f.b = cc * f.ib;
+  cross3(s.e1, cv, f.e2);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) zv[k] = cv[k] * nz;
-  cross3(yv, zv, xv);
-  f.b = dot3(xv, F);
-  const N Y0 = dot3(yv, F);
-  f.r0 = sqrt_n(dot3(F, F));
-  const N ir0 = rcp_n(f.r0);
+  for (int k = 0; k < 3; ++k) f.e2[k] *= f.ib;
+}
+
+// The set-up's adjoint: from those of b, r0, e1, e2 and the camera position
+// Cb (as the first chord's start), dL/d(inclination) and dL/d(distance): about
+// a hundred FP64 operations, a third of the set-up in forward mode along the
+// two parameters.
+__device__ inline void frame_adjoint(const DiffScene& s, int px, int py, const Frame& f,
+                                     double bb, double r0b, const double* e1b,
+                                     const double* e2b, const double* Cb, double* gi,
+                                     double* gd) {
+  const Line l = pixel_line(s, px, py);
+  double yv[3], zv[3], e1t[3], zb[3], cb[3], pb[3], yb[3], Fb[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) yv[k] = l.dv[k] * l.ny;
+  cross3(f.e2, s.e1, zv);  // e2 = e1 x zv
+  cross3(zv, e2b, e1t);
+  cross3(e2b, s.e1, zb);
+  const double zz = dot3(zv, zb);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    f.e1[k] = F[k] * ir0;
-    f.e2[k] = (xv[k] * Y0 - yv[k] * f.b) * ir0;
+    e1t[k] += e1b[k];
+    cb[k] = bb * zv[k] + (zb[k] - zv[k] * zz) * f.ib;  // zv = cv / b, b = |cv|
+  }
+  cross3(yv, cb, pb);  // cv = pv x yv
+  cross3(cb, l.pv, yb);
+  const double yy = dot3(yv, yb), ee = dot3(s.e1, e1t);
+  const double sx = s.W / 2.0 - px, sy = s.H / 2.0 - py;
+  *gi = *gd = 0.0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double db = l.ny * (yb[k] - yv[k] * yy);  // yv = dv / |dv|, dv = F - pv
+    // e1 = F / r0, r0 = |F|, F = C
+    Fb[k] = db + s.ir0 * (e1t[k] - s.e1[k] * ee) + r0b * s.e1[k] + Cb[k];
+    *gi += (pb[k] - db) * (s.fx_i[k] - s.ay_i[k] * sx - s.az_i[k] * sy) + Fb[k] * s.C_i[k];
+    *gd += Fb[k] * s.C_d[k];
   }
 }
 
@@ -193,26 +193,25 @@ template <typename T> struct DRay {
 // FP64 set-up values shared by the march and the adjoint's epilogue.  The
 // orbit angle psi is accumulated in FP64 in both precisions.
 struct Setup64 {
-  Frame<double> f;
+  Frame f;
   double ib2, l, u0, du;
   bool captured;
 };
 
 __device__ inline void diff_setup(const DiffScene& s, int px, int py, Setup64& r) {
   diff_frame(s, px, py, r.f);
-  const double b = r.f.b;
-  r.ib2 = 1.0 / (b * b);
-  r.captured = b < s.bc;
+  r.ib2 = r.f.ib * r.f.ib;
+  r.captured = r.f.b < s.bc;
   r.l = r.captured ? s.Uc : turning_point(r.ib2, s.M, s.Uc);
-  r.u0 = 1.0 / r.f.r0;
-  r.du = (r.l - r.u0) * (1.0 / s.nstep);
+  r.u0 = s.ir0;
+  r.du = (r.l - r.u0) * s.inv_nstep;
 }
 
 template <typename T>
 __device__ inline void to_ray(const DiffScene& s, const Setup64& r, DRay<T>& d) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    d.e1[k] = (T)r.f.e1[k];
+    d.e1[k] = (T)s.e1[k];
     d.e2[k] = (T)r.f.e2[k];
     d.C[k] = (T)s.C[k];
   }
@@ -220,7 +219,7 @@ __device__ inline void to_ray(const DiffScene& s, const Setup64& r, DRay<T>& d) 
   d.du = (T)r.du;
   d.h = d.du * (T)0.5;
   // z(psi) ~ cos(psi) e1_z + sin(psi) e2_z vanishes at atan2(-e1_z, e2_z) + k pi
-  const float ez1 = (float)r.f.e1[2], ez2 = (float)r.f.e2[2];
+  const float ez1 = (float)s.e1[2], ez2 = (float)r.f.e2[2];
   const float amp2 = ez1 * ez1 + ez2 * ez2;
   if (amp2 > 0.f) {
     double a = (double)atan2_fast(-ez1, ez2);
@@ -248,6 +247,18 @@ template <typename T> __device__ __forceinline__ T kappa(int j, int n) {
 }
 template <typename T> __device__ __forceinline__ T sigma(int j, int n) {
   return j < n ? (T)(n - j) : (T)(j - n) + (T)0.1;
+}
+
+// The steps' -sigma_j and kappa_j, j < kTabSteps, in LDS: the lanes of a wave
+// stand at different steps, and forming both from j takes a lane a quarter of a
+// step's instructions.  (Entries past the last step are read ahead and unused.)
+constexpr int kTabSteps = 2 * kRefSteps + 4;
+template <typename T> struct StepTab {
+  T ms, k;
+};
+template <typename T> __device__ __forceinline__ void fill_steps(StepTab<T>* tab, int n) {
+  const int j = (int)threadIdx.x;
+  if (j < kTabSteps) tab[j] = {-sigma<T>(j, n), kappa<T>(j, n)};
 }
 
 template <typename T> __device__ __forceinline__ T g_at(const DRay<T>& d, T sj) {
@@ -383,14 +394,11 @@ __device__ inline void disc_texel(const DiffScene& s, const T* q, T* c, const T*
   }
 }
 
-// Disc crossing of the chord P1 -> P2 (Annulus::Collide, vector_object.h:
-// 328-347: sign change across z = 0, crossing by linear interpolation on the
-// chord) with the soft radius window; returns the coverage (0: no crossing).
+// The point q where the line P1 -> P2 meets z = 0, by linear interpolation on
+// the chord (at the fraction sfrac of it); returns its radius.
 template <typename T>
-__device__ inline T disc_cross(const DiffScene& s, const T* P1, const T* P2, T* q, T* sfrac,
-                               T* dd) {
+__device__ inline T disc_point(const T* P1, const T* P2, T* q, T* sfrac, T* dd) {
   const T z1 = P1[2], z2 = P2[2];
-  if (!(z1 * z2 < (T)0)) return (T)0;
   const T sf = z1 * rcp(z1 - z2);
   T D[3];
 #pragma unroll
@@ -398,12 +406,21 @@ __device__ inline T disc_cross(const DiffScene& s, const T* P1, const T* P2, T* 
     D[k] = P2[k] - P1[k];
     q[k] = fma_t(sf, D[k], P1[k]);
   }
-  const T rho = sqrt_t(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
-  T g0, g1;
-  const T al = coverage<T, false>(s, rho, &g0, &g1);
   *sfrac = sf;
   *dd = sf * sf * (D[0] * D[0] + D[1] * D[1] + D[2] * D[2]);
-  return al;
+  return sqrt_t(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+}
+
+// Disc crossing of the chord P1 -> P2 (Annulus::Collide, vector_object.h:
+// 328-347: sign change across z = 0, crossing by linear interpolation on the
+// chord) with the soft radius window; returns the coverage (0: no crossing).
+template <typename T>
+__device__ inline T disc_cross(const DiffScene& s, const T* P1, const T* P2, T* q, T* sfrac,
+                               T* dd) {
+  if (!(P1[2] * P2[2] < (T)0)) return (T)0;
+  const T rho = disc_point(P1, P2, q, sfrac, dd);
+  T g0, g1;
+  return coverage<T, false>(s, rho, &g0, &g1);
 }
 
 template <typename T> struct Acc {
@@ -440,10 +457,10 @@ template <typename T> struct StepX {
   T w, x[4];
 };
 template <typename T>
-__device__ __forceinline__ StepX<T> step_x(const DRay<T>& d, int j, int n, T c3x3, T c2x2) {
-  const T sj = -sigma<T>(j, n) * d.du;
+__device__ __forceinline__ StepX<T> step_x(const DRay<T>& d, StepTab<T> st, T c3x3, T c2x2) {
+  const T sj = st.ms * d.du;
   const T w = rsq(g_at(d, sj));
-  const T kj = kappa<T>(j, n);
+  const T kj = st.k;
   const T u = fma_t(kj, d.du, d.u0);
   const T w3 = w * w * w;
   const T t = w3 * fma_t(sj, fma_t(c3x3, sj, c2x2), d.c1);
@@ -457,8 +474,18 @@ __device__ __forceinline__ StepX<T> step_x(const DRay<T>& d, int j, int n, T c3x
 //                       >= (1 - dpsi^2/8) / max(u_{j-1}, u_j)
 // does not clear the horizon radius; other chords have neither a sign change
 // of z nor a horizon entry, so skipping them changes nothing.
+//
+// A wave near the hole has some lane's chord to examine at almost every step,
+// and a 512x512 frame is one round of waves, so such waves set the launch's
+// time.  Hence each lane steps on its own, kAhead steps' G and w at a time, up
+// to its next chord to examine, and the lanes' chords are examined together:
+// as often as the ray with the most of them needs.  At 512x512 with every lane
+// at the same step: forward 32.7 us, forward and adjoint 46; this way, with the
+// step table, the closed-form frame and the waves' priority: 18.3 and 29.
+constexpr int kAhead = 4;
 template <typename T, bool RECORD>
-__device__ inline void diff_march(const DiffScene& s, const DRay<T>& d, Rec<T> rec, Acc<T>& a) {
+__device__ inline void diff_march(const DiffScene& s, const DRay<T>& d, const StepTab<T>* tab,
+                                  Rec<T> rec, Acc<T>& a) {
   a.rgb[0] = a.rgb[1] = a.rgb[2] = (T)0;
   a.tr = (T)1;
   a.cls = BH_HIT_NONE;
@@ -475,47 +502,74 @@ __device__ inline void diff_march(const DiffScene& s, const DRay<T>& d, Rec<T> r
   const T Rh = (T)s.Rh;
   const T Rh_hi = (T)(s.Rh * (1.0 + 1e-5));
   T P1[3] = {d.C[0], d.C[1], d.C[2]};
-  bool have1 = true;  // P1 holds the point of step j - 1
-  double psi = 0.0;
+  int at = 1;  // P1 is the start of chord `at`
+  double psi = 0.0, psi_prev = 0.0;
   double a_ev = d.a0 - d.guard;
-  T wp = (T)0, u_prev = d.u0;
+  T wp = (T)0, u = d.u0, u_prev = d.u0;
   T sx[4] = {(T)0, (T)0, (T)0, (T)0};  // RECORD: prefix sums of the StepX factors
   const T c3x3 = (T)3 * d.c3, c2x2 = (T)2 * d.c2;
-  for (int j = 1; j <= 2 * n - 1; ++j) {
-    if (j > n && d.captured) {
-      // chord to the centre: the horizon is entered, the disc plane is not
-      // crossed (n.(B - B) = 0)
-      if (a.cls == BH_HIT_NONE) a.cls = BH_HIT_HORIZON;
-      a.tr = (T)0;
-      break;
-    }
-    const T sj = -sigma<T>(j, n) * d.du;
-    const T w = rsq(g_at(d, sj));
-    const T dpsi = (wp + w) * d.h;
-    const double psi_prev = psi;
-    psi += (double)dpsi;
-    wp = w;
-    const T kj = kappa<T>(j, n);
-    const T u = fma_t(kj, d.du, d.u0);
-    if (RECORD) {
-      const T w3 = w * w * w;
-      const T t = w3 * fma_t(sj, fma_t(c3x3, sj, c2x2), d.c1);
-      sx[0] += t;
-      sx[1] = fma_t(kj, t, sx[1]);
-      sx[2] = fma_t(w3, u * u * u, sx[2]);
-      sx[3] += w3;
-    }
-    const T umax = u > u_prev ? u : u_prev;
-    const bool need_h = !(dpsi < (T)3) || fma_t(-dpsi * dpsi, (T)0.125, (T)1) <= Rh_hi * umax;
-    const bool need_d = psi >= a_ev;
-    if (need_h || need_d) {
+  const int last = d.captured ? n : 2 * n - 1;
+  bool live = true, need_h = false, need_d = false;
+  int j = 1;
+#pragma unroll 1
+  do {
+    bool wait = !live;
+#pragma unroll 1
+    do {
+      if (!wait) {
+        T sk[kAhead], kj[kAhead], w[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+          const StepTab<T> t = tab[j + k];
+          sk[k] = t.ms * d.du;
+          kj[k] = t.k;
+          w[k] = rsq(g_at(d, sk[k]));
+        }
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+          if (!wait && j <= last) {
+            const T dpsi = (wp + w[k]) * d.h;
+            psi_prev = psi;
+            psi += (double)dpsi;
+            wp = w[k];
+            u_prev = u;
+            u = fma_t(kj[k], d.du, d.u0);
+            if (RECORD) {
+              const T w3 = w[k] * w[k] * w[k];
+              const T t = w3 * fma_t(sk[k], fma_t(c3x3, sk[k], c2x2), d.c1);
+              sx[0] += t;
+              sx[1] = fma_t(kj[k], t, sx[1]);
+              sx[2] = fma_t(w3, u * u * u, sx[2]);
+              sx[3] += w3;
+            }
+            const T umax = u > u_prev ? u : u_prev;
+            need_h = !(dpsi < (T)3) || fma_t(-dpsi * dpsi, (T)0.125, (T)1) <= Rh_hi * umax;
+            need_d = psi >= a_ev;
+            wait = need_h || need_d;
+            if (!wait) ++j;
+          }
+        }
+        if (j > last) {
+          if (d.captured) {
+            // chord to the centre: the horizon is entered, the disc plane is
+            // not crossed (n.(B - B) = 0)
+            if (a.cls == BH_HIT_NONE) a.cls = BH_HIT_HORIZON;
+            a.tr = (T)0;
+          }
+          wait = true;
+          live = false;
+        }
+      }
+    } while (__any(!wait));
+    if (live) {
       T cs, sn;
-      if (!have1) orbit_point(d, psi_prev, rcp(u_prev), P1, &cs, &sn);
+      if (at != j) orbit_point(d, psi_prev, rcp(u_prev), P1, &cs, &sn);
       T P2[3];
       orbit_point(d, psi, rcp(u), P2, &cs, &sn);
       T dh = (T)0, q[3], sf, dd;
       const bool hh = need_h && seg_horizon(P1, P2, Rh, &dh);
-      const T al = disc_cross(s, P1, P2, q, &sf, &dd);
+      T al = (T)0;  // (before the next crossing z keeps its sign)
+      if (need_d) al = disc_cross(s, P1, P2, q, &sf, &dd);
       if (al > (T)0 && (!hh || dd < dh)) {
         T c[3];
         disc_texel<T, false>(s, q, c, nullptr, nullptr);
@@ -542,22 +596,20 @@ __device__ inline void diff_march(const DiffScene& s, const DRay<T>& d, Rec<T> r
         a.tr = a.tr * ((T)1 - al);
         if (a.cls == BH_HIT_NONE) a.cls = BH_HIT_DISC;
         ++a.n;
-        if (!(a.tr > (T)0)) break;
+        live = a.tr > (T)0;
       }
-      if (hh) {
+      if (live && hh) {
         if (a.cls == BH_HIT_NONE) a.cls = BH_HIT_HORIZON;
         a.tr = (T)0;
-        break;
+        live = false;
       }
 #pragma unroll
       for (int k = 0; k < 3; ++k) P1[k] = P2[k];
-      have1 = true;
+      ++j;
+      at = j;
       if (need_d) a_ev = next_crossing(d, psi);
-    } else {
-      have1 = false;
     }
-    u_prev = u;
-  }
+  } while (__any(live));
 }
 
 // Adjoint of P = r (cos(psi) e1 + sin(psi) e2), r = 1/u.
@@ -592,6 +644,9 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
   __shared__ T rec_ps[ADJ ? 4 * kMaxRec * kThreads : 1];
   __shared__ double red[ADJ ? kPartial * (kThreads / 64) : 1];
   const int tid = threadIdx.x;
+  __shared__ StepTab<T> tab[kTabSteps];
+  fill_steps(tab, s.nstep);
+  __syncthreads();
   const int px = blockIdx.x * kTile + (tid & (kTile - 1));
   const int py = blockIdx.y * kTile + (tid / kTile);
   const bool inside = px < s.W && py < s.H;
@@ -600,11 +655,15 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
     const size_t idx = (size_t)py * s.W + px;
     Setup64 su;
     diff_setup(s, px, py, su);
+    // the waves near the hole have the most chords to examine and end last:
+    // they issue first (forward 22.0 -> 18.8 us at 512x512, where all waves are
+    // resident; the adjoint, in two rounds of waves, gains nothing by it)
+    if (!ADJ && __any(su.f.b < 1.3 * s.bc)) __builtin_amdgcn_s_setprio(3);
     DRay<T> d;
     to_ray(s, su, d);
     Acc<T> a;
     const Rec<T> rec{rec_psi + tid, rec_tr + tid, rec_ps + tid};
-    diff_march<T, ADJ>(s, d, rec, a);
+    diff_march<T, ADJ>(s, d, tab, rec, a);
     if (rgb_out) {
       rgb_out[3 * idx + 0] = (float)a.rgb[0];
       rgb_out[3 * idx + 1] = (float)a.rgb[1];
@@ -614,7 +673,6 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
     if (ADJ) g_ov = a.overflow ? 1.0 : 0.0;
     if (ADJ && a.mask) {
       const T gb[3] = {(T)grad_rgb[3 * idx], (T)grad_rgb[3 * idx + 1], (T)grad_rgb[3 * idx + 2]};
-      const int n = s.nstep;
       T B[3] = {(T)0, (T)0, (T)0};
       T e1b[3] = {(T)0, (T)0, (T)0}, e2b[3] = {(T)0, (T)0, (T)0}, Cb[3] = {(T)0, (T)0, (T)0};
       T hb = (T)0, u0b = (T)0, dub = (T)0, Mb = (T)0, ib2b = (T)0, rinb = (T)0;
@@ -627,8 +685,9 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
       while (mask) {
         const int j = 63 - __builtin_clzll(mask);
         mask &= ~(1ull << j);
-        const StepX<T> xj = step_x(d, j, n, c3x3, c2x2);
-        const StepX<T> xi = step_x(d, j > 1 ? j - 1 : 1, n, c3x3, c2x2);  // used for j > 1
+        const StepTab<T> tj = tab[j], ti = tab[j > 1 ? j - 1 : 1];
+        const StepX<T> xj = step_x(d, tj, c3x3, c2x2);
+        const StepX<T> xi = step_x(d, ti, c3x3, c2x2);  // used for j > 1
         double ps_a, ps_b;
         if constexpr (Rec<T>::kPsi == 1) {
           ps_b = (double)rec.psi[k * kThreads] * (1.0 / kPsiUnit);
@@ -642,21 +701,22 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
 #pragma unroll
         for (int q = 0; q < 4; ++q) S0[q] = rec.ps[(4 * k + q) * kThreads];
         --k;
-        const T uj = fma_t(kappa<T>(j, n), d.du, d.u0);
+        const T uj = fma_t(tj.k, d.du, d.u0);
         T P1[3], P2[3], ca = (T)0, sa = (T)0, ra = (T)0, cb, sb;
         if (j == 1) {
 #pragma unroll
           for (int m = 0; m < 3; ++m) P1[m] = d.C[m];
         } else {
-          ra = rcp(fma_t(kappa<T>(j - 1, n), d.du, d.u0));
+          ra = rcp(fma_t(ti.k, d.du, d.u0));
           orbit_point(d, ps_a, ra, P1, &ca, &sa);
         }
         const T rb = rcp(uj);
         orbit_point(d, ps_b, rb, P2, &cb, &sb);
+        // (the recorded angle is rounded, so a crossing at the very end of its
+        // chord may lie just off the chord formed here: no sign test)
         T q[3], sf, dd;
         const T z1 = P1[2], z2 = P2[2];
-        disc_cross(s, P1, P2, q, &sf, &dd);
-        const T rho = sqrt_t(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+        const T rho = disc_point(P1, P2, q, &sf, &dd);
         T da_rho, da_rin;
         const T al = coverage<T, true>(s, rho, &da_rho, &da_rin);
         T c[3], cw[3], qb[3];
@@ -693,7 +753,7 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
         T phb, ub;
         point_adjoint(d, P2b, cb, sb, rb, e1b, e2b, &phb, &ub);
         u0b += ub;
-        dub = fma_t(kappa<T>(j, n), ub, dub);
+        dub = fma_t(tj.k, ub, dub);
         T S1[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -708,7 +768,7 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
           // the start point: angle psi_{j-1} (injection m = j - 1)
           point_adjoint(d, P1b, ca, sa, ra, e1b, e2b, &phb, &ub);
           u0b += ub;
-          dub = fma_t(kappa<T>(j - 1, n), ub, dub);
+          dub = fma_t(ti.k, ub, dub);
 #pragma unroll
           for (int m = 0; m < 4; ++m) wx[m] = fma_t(phb, (T)2 * S1[m] - xi.x[m], wx[m]);
           hb = fma_t(phb, (T)ps_a * ih, hb);
@@ -723,29 +783,35 @@ __global__ __launch_bounds__(kThreads, (ADJ && sizeof(T) == 4) ? 3 : 1) void dif
       // epilogue in FP64: h = du/2, du = (l - u0)/n, l(M, 1/b^2), set-up
       // (psi starts at 0 whatever the parameters, so A_1 goes nowhere)
       double dub64 = (double)dub + 0.5 * (double)hb;
-      const double lb = dub64 / n;
-      double u0b64 = (double)u0b - lb;
+      const double lb = dub64 * s.inv_nstep;
+      const double u0b64 = (double)u0b - lb;
       double Mb64 = (double)Mb, ib2b64 = (double)ib2b;
-      const double M = s.M, l = su.l;
+      const double l = su.l;
       if (su.captured) {
-        Mb64 += lb * (-1.0 / (3.0 * M * M));
+        Mb64 -= lb * (3.0 * s.Uc * s.Uc);  // l = 1/(3M)
       } else {
-        const double Gu = l * __builtin_fma(6.0 * M, l, -2.0);
-        Mb64 += lb * (-2.0 * l * l * l / Gu);
-        ib2b64 += lb * (-1.0 / Gu);
+        const double Gu = l * __builtin_fma(6.0 * s.M, l, -2.0);
+        const double k = lb / Gu;
+        Mb64 -= k * (2.0 * l * l * l);
+        ib2b64 -= k;
       }
-      const double b = su.f.b, r0 = su.f.r0;
-      const double bb = ib2b64 * (-2.0 / (b * b * b));
-      const double r0b = -u0b64 / (r0 * r0);
-      Frame<D2> fd;
-      diff_frame(s, px, py, fd);
-      double gi = bb * fd.b.i + r0b * fd.r0.i;
-      double gd = bb * fd.b.d + r0b * fd.r0.d;
+      // the frame again rather than kept through the march: an empty asm
+      // statement hides from the compiler that the pixel is the same
+      int px2 = px;
+      __asm__ volatile("" : "+v"(px2));
+      Frame f;
+      diff_frame(s, px2, py, f);
+      const double bb = -2.0 * ib2b64 * (f.ib * f.ib) * f.ib;
+      const double r0b = -u0b64 * s.ir0 * s.ir0;
+      double e1d[3], e2d[3], Cd[3];
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
-        gi += (double)e1b[m] * fd.e1[m].i + (double)e2b[m] * fd.e2[m].i + (double)Cb[m] * s.C_i[m];
-        gd += (double)e1b[m] * fd.e1[m].d + (double)e2b[m] * fd.e2[m].d + (double)Cb[m] * s.C_d[m];
+        e1d[m] = (double)e1b[m];
+        e2d[m] = (double)e2b[m];
+        Cd[m] = (double)Cb[m];
       }
+      double gi, gd;
+      frame_adjoint(s, px2, py, f, bb, r0b, e1d, e2d, Cd, &gi, &gd);
       g_rs = 0.5 * Mb64;  // M = r_s / 2
       g_in = gi;
       g_di = gd;

@@ -9,6 +9,10 @@
 
 namespace bh {
 
+// The step count of the reference's step rule (blackhole_solution_test.cc
+// and the shipped scene): the FP32 march has an instance compiled for it.
+constexpr int kRefSteps = 20;
+
 // Texture in HBM: one packed little-endian RGBA word per texel (channel 0 in
 // the low byte), so every lookup is one aligned 4-byte load.
 struct DevTex {
@@ -243,7 +247,9 @@ struct DiffScene {
   double fx[3], fx_i[3];              // axis_x * focal length (focus vector)
   double ay[3], ay_i[3];              // axis_y
   double az[3], az_i[3];              // axis_z
+  double ir0, e1[3];                  // 1/|C| and C/|C|
   double M, bc, Rh, Uc;               // mass, 3 sqrt(3) M, 2M, 1/(3M)
+  double inv_nstep;                   // 1 / nstep
   double r_in, r_out, edge;           // disc radii and soft-edge width
   double half, uscale, vscale;        // texture square half side; cols, rows / (2 half)
   DevTex tex;                         // disc texture (data null: black disc)

@@ -483,10 +483,6 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
 // steps of a block take one event check between them, which keeps the
 // exec-mask bookkeeping of the hot loop to a handful of scalar instructions
 // per block.
-// The step count of the reference's step rule (blackhole_solution_test.cc
-// and the shipped scene): the FP32 march has an instance compiled for it.
-constexpr int kRefSteps = 20;
-
 template <typename T, bool ESCAPE, bool SPH = false, int NS = 0>
 __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, double first_aa,
                              double du64, MarchOut<T>& o) {

@@ -1,6 +1,6 @@
 // bh_math.h — small device math shared by the march kernels: precision-
 // generic wrappers of the hardware reciprocal / rsqrt / sqrt, FP32 and FP64
-// sin/cos of bounded arguments, an FP32 atan2, and forward-mode dual numbers.
+// sin/cos of bounded arguments and an FP32 atan2.
 #pragma once
 
 #include "bh_fp64.h"
