@@ -153,6 +153,10 @@ SIGNATURES = {
                                     C.POINTER(C.c_double)]),
     "bh_diff_render_device": (C.c_int, [P, C.POINTER(DiffParams), C.c_int, P, P]),
     "bh_diff_adjoint_device": (C.c_int, [P, C.POINTER(DiffParams), C.c_int, P, P, P, P, P]),
+    "bh_diff_render_stream": (C.c_int, [P, P, C.POINTER(DiffParams), C.c_int, P, P]),
+    "bh_diff_work_bytes": (C.c_size_t, [C.c_int, C.c_int]),
+    "bh_diff_adjoint_stream": (C.c_int, [P, P, C.POINTER(DiffParams), C.c_int, P, P, P, P, P, P,
+                                         C.c_size_t]),
     "bh_diff_time": (C.c_int, [P, C.POINTER(DiffParams), C.c_int, C.c_int,
                                C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "bh_render_flat": (C.c_int, [P, C.POINTER(FlatScene), C.POINTER(Outputs)]),

@@ -47,6 +47,8 @@ struct bh_ctx {
   int wall_khz = 0;
   void* noalloc = nullptr;  // this device's allocation-free scratch array
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
+  hipEvent_t ev_order = nullptr;  // orders a caller's stream after the context's
+  bool other_streams = false;  // a call has put work on a caller's stream
   char name[256] = {0};
   int n_cu = 0, clock_khz = 0;
 };
@@ -668,6 +670,59 @@ int build_diff(bh_ctx* ctx, const bh_diff_params* p, int precision, bh::DiffScen
   return BH_OK;
 }
 
+size_t diff_work(int W, int H) {
+  return (size_t)bh::diff_partial_blocks(W, H) * 5 * sizeof(double);
+}
+
+// Readies the context for a call on a stream of the caller's: the stream waits
+// for what the context's own stream still holds.  (A capture cannot wait for
+// work outside it.)
+void enter_stream(bh_ctx* ctx, hipStream_t st) {
+  if (st == ctx->stream) return;
+  ctx->other_streams = true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return;
+  }
+  if (hipStreamQuery(ctx->stream) == hipSuccess) return;
+  (void)hipGetLastError();
+  if (hipEventRecord(ctx->ev_order, ctx->stream) != hipSuccess ||
+      hipStreamWaitEvent(st, ctx->ev_order, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(ctx->stream);
+  }
+}
+
+// Waits for all work the context's calls have put on the device.
+hipError_t context_idle(bh_ctx* ctx) {
+  if (!ctx->other_streams) return hipStreamSynchronize(ctx->stream);
+  const hipError_t e = hipDeviceSynchronize();
+  if (e == hipSuccess) ctx->other_streams = false;
+  return e;
+}
+
+int diff_render_on(bh_ctx* ctx, hipStream_t st, const bh_diff_params* p, int precision,
+                   float* rgb, uint8_t* hit) {
+  bh::DiffScene d;
+  int rc = build_diff(ctx, p, precision, &d);
+  if (rc) return rc;
+  (void)hipSetDevice(ctx->device);
+  enter_stream(ctx, st);
+  HIP_TRY(ctx, bh::launch_diff_forward(d, precision == BH_PREC_FP64, rgb, hit, st));
+  return BH_OK;
+}
+
+int diff_adjoint_scene(bh_ctx* ctx, const bh_diff_params* p, int precision, const float* grad_rgb,
+                       double* grad_out, bh::DiffScene* d) {
+  if (!grad_rgb || !grad_out)
+    return fail(ctx, BH_ERR_INVALID_ARG, "grad_rgb and grad_out are required");
+  int rc = build_diff(ctx, p, precision, d);
+  if (rc) return rc;
+  (void)hipSetDevice(ctx->device);
+  return BH_OK;
+}
+
 // Fused path launches: the queue counts cleared and every frame's march in one
 // launch (up to 1024 frames each), then every frame's FP64 band pass in one launch.
 constexpr int kFramesPerLaunch = 1024;
@@ -730,6 +785,7 @@ int bh_ctx_create(int device, bh_ctx** out) {
     (void)hipEventCreate(&c->ev0);
     (void)hipEventCreate(&c->ev1);
     (void)hipEventCreate(&c->ev2);
+    (void)hipEventCreateWithFlags(&c->ev_order, hipEventDisableTiming);
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
       std::snprintf(c->name, sizeof c->name, "%s (%s)", prop.name, prop.gcnArchName);
@@ -749,7 +805,7 @@ int bh_ctx_create(int device, bh_ctx** out) {
 void bh_ctx_destroy(bh_ctx* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
-  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  if (ctx->stream) (void)context_idle(ctx);
   for (auto& t : ctx->tex)
     if (t.d) (void)hipFree(t.d);
   for (DevBuf* b : {&ctx->scene, &ctx->rgb, &ctx->hit, &ctx->phi, &ctx->hitpt, &ctx->steps,
@@ -760,6 +816,7 @@ void bh_ctx_destroy(bh_ctx* ctx) {
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev2) (void)hipEventDestroy(ctx->ev2);
+  if (ctx->ev_order) (void)hipEventDestroy(ctx->ev_order);
   if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   delete ctx;
@@ -803,7 +860,7 @@ int bh_ctx_set_stream(bh_ctx* ctx, void* stream) {
 int bh_synchronize(bh_ctx* ctx) {
   return guarded(ctx, [&]() -> int {
     if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    HIP_TRY(ctx, context_idle(ctx));
     return BH_OK;
   });
 }
@@ -829,7 +886,7 @@ int bh_texture_set(bh_ctx* ctx, int slot, const bh_image* img) {
                   ((C == 4 ? (uint32_t)p[3] : 255u) << 24);
     }
     DeviceTexture& t = ctx->tex[slot];
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    HIP_TRY(ctx, context_idle(ctx));
     if (t.d && (size_t)t.rows * t.cols != n) {
       (void)hipFree(t.d);
       t.d = nullptr;
@@ -848,7 +905,7 @@ int bh_texture_clear(bh_ctx* ctx, int slot) {
     if (slot < 0 || slot >= BH_MAX_TEXTURES) return fail(ctx, BH_ERR_INVALID_ARG, "texture slot out of range");
     DeviceTexture& t = ctx->tex[slot];
     if (t.d) {
-      HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+      HIP_TRY(ctx, context_idle(ctx));
       (void)hipFree(t.d);
     }
     t = DeviceTexture{};
@@ -1279,12 +1336,15 @@ int bh_diff_render_device(bh_ctx* ctx, const bh_diff_params* p, int precision, f
                           uint8_t* hit_out) {
   return guarded(ctx, [&]() -> int {
     if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
-    bh::DiffScene d;
-    int rc = build_diff(ctx, p, precision, &d);
-    if (rc) return rc;
-    (void)hipSetDevice(ctx->device);
-    HIP_TRY(ctx, bh::launch_diff_forward(d, precision == BH_PREC_FP64, rgb_out, hit_out, ctx->stream));
-    return BH_OK;
+    return diff_render_on(ctx, ctx->stream, p, precision, rgb_out, hit_out);
+  });
+}
+
+int bh_diff_render_stream(bh_ctx* ctx, void* stream, const bh_diff_params* p, int precision,
+                          float* rgb_out, uint8_t* hit_out) {
+  return guarded(ctx, [&]() -> int {
+    if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
+    return diff_render_on(ctx, (hipStream_t)stream, p, precision, rgb_out, hit_out);
   });
 }
 
@@ -1293,15 +1353,37 @@ int bh_diff_adjoint_device(bh_ctx* ctx, const bh_diff_params* p, int precision,
                            double* grad_out, uint32_t* overflow_out) {
   return guarded(ctx, [&]() -> int {
     if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
-    if (!grad_rgb || !grad_out) return fail(ctx, BH_ERR_INVALID_ARG, "grad_rgb and grad_out are required");
     bh::DiffScene d;
-    int rc = build_diff(ctx, p, precision, &d);
+    int rc = diff_adjoint_scene(ctx, p, precision, grad_rgb, grad_out, &d);
     if (rc) return rc;
-    (void)hipSetDevice(ctx->device);
-    const size_t nb = (size_t)bh::diff_partial_blocks(d.W, d.H);
-    if ((rc = ensure(ctx, ctx->dpart, nb * 5 * sizeof(double)))) return rc;
+    if ((rc = ensure(ctx, ctx->dpart, diff_work(d.W, d.H)))) return rc;
     HIP_TRY(ctx, bh::launch_diff_adjoint(d, precision == BH_PREC_FP64, grad_rgb, rgb_out, hit_out,
-                                         (double*)ctx->dpart.p, grad_out, overflow_out, ctx->stream));
+                                         (double*)ctx->dpart.p, grad_out, overflow_out,
+                                         ctx->stream));
+    return BH_OK;
+  });
+}
+
+size_t bh_diff_work_bytes(int width, int height) {
+  return width > 0 && height > 0 ? diff_work(width, height) : 0;
+}
+
+int bh_diff_adjoint_stream(bh_ctx* ctx, void* stream, const bh_diff_params* p, int precision,
+                           const float* grad_rgb, float* rgb_out, uint8_t* hit_out,
+                           double* grad_out, uint32_t* overflow_out, void* work,
+                           size_t work_bytes) {
+  return guarded(ctx, [&]() -> int {
+    if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
+    bh::DiffScene d;
+    int rc = diff_adjoint_scene(ctx, p, precision, grad_rgb, grad_out, &d);
+    if (rc) return rc;
+    if (!work || ((uintptr_t)work & 7) || work_bytes < diff_work(d.W, d.H))
+      return fail(ctx, BH_ERR_INVALID_ARG,
+                  "work must be 8-aligned and bh_diff_work_bytes(width, height) long");
+    enter_stream(ctx, (hipStream_t)stream);
+    HIP_TRY(ctx, bh::launch_diff_adjoint(d, precision == BH_PREC_FP64, grad_rgb, rgb_out, hit_out,
+                                         (double*)work, grad_out, overflow_out,
+                                         (hipStream_t)stream));
     return BH_OK;
   });
 }

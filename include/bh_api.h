@@ -395,6 +395,19 @@ int bh_diff_render_device(bh_ctx* ctx, const bh_diff_params* p, int precision,
 int bh_diff_adjoint_device(bh_ctx* ctx, const bh_diff_params* p, int precision,
                            const float* grad_rgb, float* rgb_out, uint8_t* hit_out,
                            double* grad_out, uint32_t* overflow_out);
+/* The two calls on a stream of the caller's (hipStream_t; NULL is the null
+ * stream) in place of the context's: a caller whose buffers belong to that
+ * stream needs no events around the call.  They start after the work that the
+ * context's stream holds (not under capture), and the context keeps nothing of
+ * them: work is the caller's, bh_diff_work_bytes long and 8-aligned, and in use
+ * until the call's work has ended. */
+int bh_diff_render_stream(bh_ctx* ctx, void* stream, const bh_diff_params* p, int precision,
+                          float* rgb_out, uint8_t* hit_out);
+size_t bh_diff_work_bytes(int width, int height);
+int bh_diff_adjoint_stream(bh_ctx* ctx, void* stream, const bh_diff_params* p, int precision,
+                           const float* grad_rgb, float* rgb_out, uint8_t* hit_out,
+                           double* grad_out, uint32_t* overflow_out, void* work,
+                           size_t work_bytes);
 /* Average ms of the forward kernel and of the forward+adjoint kernel over
  * iters back-to-back launches (HIP events on the context stream). */
 int bh_diff_time(bh_ctx* ctx, const bh_diff_params* p, int precision, int iters,
