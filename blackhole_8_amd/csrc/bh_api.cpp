@@ -12,6 +12,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <string>
+#include <limits>
 #include <vector>
 
 #include "bh_api.h"
@@ -291,6 +292,24 @@ int build_scene(bh_ctx* ctx, const bh_scene* sc, const bh_options* opt_in, DevSc
   d->Rhf = (float)d->Rh;
   d->u0f = (float)d->u0;
   d->ktf = (float)d->nstep - 0.1f;
+  // The reach of the disc, and the b^2 beyond which a ray's chords all pass it
+  // and the horizon.  A ray turns at r_t with b = r_t / sqrt(1 - 2M/r_t); its
+  // largest increment d is that into the approach point, where
+  // G(l - s) >= 2 l (1 - 3Ml) s (1 - 0.03) at s = du/10 <= l / (10 nstep), so
+  // d <= du / sqrt(G) gives d^2 <= 5.2 / (nstep (1 - 3M/r_t)), and no chord
+  // comes nearer than r_t (1 - d^2/8).  b^2 >= 1.6 b_c^2 puts r_t beyond
+  // 5.1M (1 - 3M/r_t >= 0.41), which clears the horizon from 5 steps on.
+  d->reach = d->has_disc && d->r_out >= 0.0 ? (float)(d->r_out * (1.0 + 1e-4)) : 0.f;
+  d->far2 = std::numeric_limits<double>::infinity();
+  if (d->nstep >= 5) {
+    d->far2 = 1.6 * d->bc2;
+    const double R = d->reach;
+    if (R > 0.0) {
+      const double dl = std::max(1.0 - d->M3 / R, 0.41);
+      const double rt = R / (1.0 - 5.2 / (d->nstep * dl) / 8.0);
+      if (rt > d->M3) d->far2 = std::max(d->far2, rt * rt / (1.0 - d->M2 / rt));
+    }
+  }
   d->alpha_f = d->nf[0] * d->e1f[0] + d->nf[1] * d->e1f[1] + d->nf[2] * d->e1f[2];
   d->r_in2 = d->r_in > 0.0 ? (float)(d->r_in * d->r_in) : -1.0f;
   d->r_out2 = d->r_out >= 0.0 ? (float)(d->r_out * d->r_out) : -1.0f;

@@ -338,7 +338,7 @@ __device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, uint3
   }
   const size_t idx = (size_t)y * s.W + x;
   RaySetup r;
-  setup_ray(s, x, y, false, r);
+  setup_ray32<ESCAPE, SPH>(s, b.outs[sc], x, y, r);
   const bool band = r.band && !r.degenerate;
   if (!push_band(b, band, id, 0u, false) && band) return false;
   const float phi0 = phi0_of(b.outs[sc], r);
@@ -346,12 +346,14 @@ __device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, uint3
   bool sredo = false;
   if (r.degenerate) {
     degenerate_out(mo);
+  } else if (r.over) {
+    over_out(s, r, mo);
   } else {
     Lane<float> L;
     const double du = (r.l - s.u0) * s.inv_nstep;
     setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
     if constexpr (SPH) setup_spheres32(s, r, L);
-    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, mo);
+    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(b.outs[sc]), mo);
     if constexpr (SPH) sredo = L.sredo;
   }
   const bool redo = finish_ray<ESCAPE>(s, b.outs[sc], idx, r, mo, phi0) || sredo;

@@ -60,6 +60,7 @@ struct DevScene {
   // pv x F = pxC - sx pxCy - sy pxCz and dv . F = pxF[0] + sx pxF[1] + sy pxF[2]
   double pxD[3], pxC[3], pxCy[3], pxCz[3], pxF[3];
   double bc2, lo2, hi2;   // b_c^2 and the band's bounds on b^2
+  double far2;            // an escaping ray with b^2 > far2 meets neither disc nor horizon
   double Uc;              // 1/(3M)
   double r02;             // |C - B|^2
   double cell, inv_cell;  // SolveG grid: (1/(3M) - l0) / 2^20 and its inverse
@@ -67,6 +68,7 @@ struct DevScene {
   double M2, M3, M6;      // 2M, 3M, 6M
   float Rhf, u0f;         // R_h and u0 in FP32
   float ktf;              // nstep - 0.1 in FP32
+  float reach;            // r_outer (1 + 1e-4) in FP32, 0 without a disc
   float e1f[3];           // F / |F|
   float nf[3];            // disc normal
   float alpha_f;          // n . e1

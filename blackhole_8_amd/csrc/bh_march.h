@@ -483,9 +483,23 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
 // steps of a block take one event check between them, which keeps the
 // exec-mask bookkeeping of the hot loop to a handful of scalar instructions
 // per block.
+//
+// brief (frames whose swept angle is not asked for, discs and holes only): a
+// ray that can meet nothing any more ends at once, with the step count that
+// it would end with:
+//  - at the approach point, if twice the angle swept so far does not reach the
+//    next crossing: the outbound points lie 0.1 du nearer the turning point
+//    on their cubic's falling side, w(sigma + 0.1) <= w(sigma), so the way out
+//    sweeps at most what the way in did (2e-5 covers FP32 rounding);
+//  - at the end of an outbound block whose last point lies beyond the disc
+//    (DevScene.reach, 1e-4 outside it): the radii grow and the increments
+//    shrink from there, so no later chord comes nearer than
+//    r cos(d/2) >= r (1 - d^2/8).
+// A wave of a disc seen from 20 r_s at 10 degrees took 27.3 steps on average
+// and takes 21.7.
 template <typename T, bool ESCAPE, bool SPH = false, int NS = 0>
 __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, double first_aa,
-                             double du64, MarchOut<T>& o) {
+                             double du64, bool brief, MarchOut<T>& o) {
   // NS > 0: the scene's nstep, known at compile time: the blocks unroll, and
   // their step values and chord ends become literal operands (no per-step
   // integer-to-float conversion, no loop bookkeeping)
@@ -515,6 +529,12 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
     if constexpr (SPH) L.a_sph = 1e308;  // no sphere tests either once ended
   };
   auto armed = [&]() { return L.phi_safe < kInf; };
+  constexpr bool kBrief = !ESCAPE && !SPH;
+  // no chord of increment <= d from radius >= 1/u can meet the disc or the
+  // horizon
+  auto clear = [&](float u, float d) {
+    return d <= L.phi_safe && u * s.reach < __builtin_fmaf(d * d, -0.125f, 1.f);
+  };
   auto step = [&](int n, T G, T ka, T kb, bool force) {
     if (march_step<T, DevScene, SPH>(s, L, st, first_aa, G, ka, kb, force, o.hit)) end_ray(n);
   };
@@ -569,7 +589,8 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
     const T dlast = wk[K - 2] + wk[K - 1];
     // the last increment is read after the block only by end_ray, which
     // an outbound block's successor may call before stepping
-    if (inbound || n0 + 2 * K > 2 * nstep) st.d = dlast;
+    // (or by the brief march's test)
+    if (kBrief || inbound || n0 + 2 * K > 2 * nstep) st.d = dlast;
     const float dmax = inbound ? dlast : w0 + wk[0];
     bool ev = dmax > L.phi_safe || st.a >= L.a_ev;
     if constexpr (SPH) ev = ev || dmax > fmaxf(1.f, L.phi_safe) || st.a >= L.a_sph;
@@ -628,19 +649,31 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
       captured_chord<T, SPH>(s, L, st.a, o.hit);
       end_ray(nstep);
     }
+    if constexpr (kBrief) {
+      if (brief && armed() && (float)st.d <= L.phi_safe && st.a * 2.00002 < L.a_ev)
+        end_ray(2 * nstep - 1);
+    }
     if (!__any(armed())) goto done;
     // outbound: u -= du (:274-296)
+    auto beyond = [&](int m) {  // after step m
+      if constexpr (!kBrief) return false;
+      const float kb = ((float)nstep - 0.1f) - (float)(m - nstep);
+      return brief && armed() &&
+             clear(__builtin_fmaf(kb, (float)L.du, (float)L.u0), (float)st.d);
+    };
     n = nstep + 1;
     if constexpr (NS > 0) {
 #pragma unroll
       for (int b = 0; b < (NS - 1) / kB; ++b) {
         block(NS + 1 + kB * b, out_coeffs, false, std::integral_constant<int, kB>{});
+        if (beyond(NS + kB * (b + 1))) end_ray(2 * nstep - 1);
         if (!__any(armed())) goto done;
       }
       n = NS + 1 + kB * ((NS - 1) / kB);
     } else {
       for (; n + 3 < 2 * nstep; n += 4) {
         block(n, out_coeffs, false, std::integral_constant<int, 4>{});
+        if (beyond(n + 3)) end_ray(2 * nstep - 1);
         if (!__any(armed())) goto done;
       }
     }
@@ -661,6 +694,9 @@ __device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, doubl
   }
 done:;
 }
+
+// Planes that the brief march can fill: the swept angle is not among them.
+__device__ __forceinline__ bool brief_march(const DevOut& out) { return !out.phi; }
 
 // tex_index for an FP32 coordinate, without the FP64 round trip: the same
 // index for every float v (NaN -> 0; n - 1 < 2^24 is exact in FP32).
@@ -881,10 +917,15 @@ struct RaySetup {
   double cc, dd, dF, ib2, l, first_aa;
   float e2x, e2y, e2z, sgn;
   bool degenerate, captured, band;
+  bool over;  // brief frames: the class is known without a march
 };
 
+// far2 (DevScene.far2; +inf: march every ray) and capt: an escaping ray with
+// b^2 > far2 meets nothing, and with capt the horizon class is all that is
+// asked of a captured one; such a ray ends here (r.over).
 __device__ inline void setup_ray(const DevScene& s, int x, int y, bool force_bisect,
-                                 RaySetup& r) {
+                                 RaySetup& r, double far2 = __builtin_inf(),
+                                 bool capt = false) {
   // the pixel point pv = fvB - sx vy - sy vz (relative to B) enters only
   // through dv = F - pv (along yv), cv = pv x F (|cv| = b |dv|) and dv.F,
   // each linear in (sx, sy) with coefficients formed once per frame
@@ -912,7 +953,8 @@ __device__ inline void setup_ray(const DevScene& s, int x, int y, bool force_bis
   r.e2x = r.e2y = r.e2z = 0.f;
   r.ib2 = 0.0;
   r.l = s.Uc;
-  if (r.degenerate) return;
+  r.over = !r.degenerate && !r.band && (r.captured ? capt : dF > 0.0 && cc > dd * far2);
+  if (r.degenerate || r.over) return;
   // 1 / b^2 = dd / cc: hardware reciprocal and two Newton steps (<= 2 ulp)
   double rc = __builtin_amdgcn_rcp(cc);
   rc = rc * __builtin_fma(-cc, rc, 2.0);
@@ -986,6 +1028,32 @@ __device__ inline void setup_spheres32(const DevScene& s, const RaySetup& r, Lan
 // the march so that cc and dF need not stay live through it.
 __device__ __forceinline__ float phi0_of(const DevOut& out, const RaySetup& r) {
   return (out.phi && !r.degenerate) ? (float)atan(sqrt(r.cc) / r.dF) : 0.f;
+}
+
+// The FP32 march's set-up: setup_ray with the brief frames' early ends.
+template <bool ESCAPE, bool SPH>
+__device__ __forceinline__ void setup_ray32(const DevScene& s, const DevOut& out, int x, int y,
+                                            RaySetup& r) {
+  if constexpr (ESCAPE || SPH) {
+    setup_ray(s, x, y, false, r);
+  } else {
+    const bool brief = brief_march(out);
+    setup_ray(s, x, y, false, r, brief ? s.far2 : __builtin_inf(),
+              brief && !s.has_disc && !out.steps && !out.hitpt);
+  }
+}
+
+// The outcome of a ray that ended in its set-up.
+__device__ __forceinline__ void over_out(const DevScene& s, const RaySetup& r,
+                                         MarchOut<float>& mo) {
+  mo.hit.cls = r.captured ? BH_HIT_HORIZON : BH_HIT_NONE;
+  mo.hit.obj = 0;
+  mo.hit.ang = 0.0;
+  mo.hit.hx = mo.hit.hy = 0.f;
+  mo.du64 = 0.0;
+  mo.steps = r.captured ? s.nstep : 2 * s.nstep - 1;
+  mo.a = 0.0;
+  mo.d = 0.f;
 }
 
 // Hit point, colour and output planes of one ray.  Returns true when the

@@ -56,7 +56,7 @@ __device__ __forceinline__ void march_pixel(const DevScene& s, const DevOut& out
                                             const DevQueue& q, uint32_t k, int x, int y) {
   const size_t idx = (size_t)y * s.W + x;
   RaySetup r;
-  setup_ray(s, x, y, false, r);
+  setup_ray32<ESCAPE, SPH>(s, out, x, y, r);
   // queued for the FP64 march (a full queue would march the ray here)
   if (r.band && !r.degenerate && queue_push_band(q, k, (uint32_t)idx)) return;
   const float phi0 = phi0_of(out, r);
@@ -64,12 +64,14 @@ __device__ __forceinline__ void march_pixel(const DevScene& s, const DevOut& out
   bool sredo = false;
   if (r.degenerate) {
     degenerate_out(mo);
+  } else if (r.over) {
+    over_out(s, r, mo);
   } else {
     Lane<float> L;
     const double du = (r.l - s.u0) * s.inv_nstep;
     setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
     if constexpr (SPH) setup_spheres32(s, r, L);
-    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, mo);
+    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
     if constexpr (SPH) sredo = L.sredo;
   }
   // the texel lies within the FP32 error of a texel edge (or a sphere was
