@@ -325,48 +325,95 @@ __device__ inline void run_lanes(const BatchDev& b, uint32_t waves) {
   flush(b, f);
 }
 
+// The rgb and hit planes of a wave whose 64 lanes hold a whole tile of 8x8
+// pixels at (x0, y0), v = rgb | class << 24 on every lane: 48 lanes store a
+// dword of rgb and 16 a dword of classes, in one store instruction.  The
+// stores by lane (a short and two bytes of each pixel, eight rows of scenes of
+// any width) kept the texture-address unit busy for 290 cycles a wave, which
+// bounded a batch whose rays end early: 512 scenes, 77.6 Mpixel, took 930 us
+// in the grid launch and take 758.  (A frame's waves hold 16x4 pixels at
+// aligned rows and are bound by their arithmetic; packing cost them 8%.)
+__device__ __forceinline__ void store_tile(const DevOut& out, uint32_t W, uint32_t x0, uint32_t y0,
+                                           uint32_t v) {
+  const uint32_t t = (uint32_t)lane_id();
+  // classes of four neighbours in their first lane
+  const uint32_t v1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true);
+  const uint32_t h1 = __builtin_amdgcn_perm(v1, v, 0x0c0c0703u);
+  const uint32_t h2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h1, 0x4E, 0xf, 0xf, true);
+  const uint32_t h = __builtin_amdgcn_perm(h2, h1, 0x05040100u);
+  // dword j of a row holds bytes 4j .. 4j+3: from pixel j + j/3, byte j mod 3;
+  // lane 48 + 2 row + i holds the classes 4i .. 4i+3 of a row
+  const bool rgb = t < 48u;
+  const uint32_t row = rgb ? t * 43u >> 8 : (t - 48u) >> 1;
+  const uint32_t j = rgb ? t - 6u * row : t & 1u;
+  const uint32_t k = j < 3u ? j : j - 3u;
+  const uint32_t col = rgb ? (j < 3u ? j : j + 1u) : 4u * j;
+  const int src = (int)(4u * (8u * row + col));
+  const uint32_t a = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v);
+  const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute(src + 4, (int)v);
+  const uint32_t hh = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)h);
+  const uint32_t sel = k == 0u ? 0x04020100u : k == 1u ? 0x05040201u : 0x06050402u;
+  const uint32_t word = rgb ? __builtin_amdgcn_perm(b, a, sel) : hh;
+  const uint32_t pix = (y0 + row) * W + x0;
+  const uint64_t p = (rgb ? (uint64_t)out.rgb + 3ull * pix : (uint64_t)out.hit + pix) + 4u * j;
+  // planes of any alignment; device memory, also where the pointer was loaded
+  struct __attribute__((packed)) Word { uint32_t w; };
+  using GlobalWord = __attribute__((address_space(1))) Word;
+  reinterpret_cast<GlobalWord*>(p)->w = word;
+}
+
 // Tile mode: a wave takes a whole 8x8 tile of one scene and marches it with
 // the per-frame kernel's wave-uniform loop (scene constants in scalar
 // registers).  Returns whether this lane's ray was finished here (not queued
 // for the band pass).
 template <bool ESCAPE, bool SPH, int NS = 0>
-__device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, uint32_t sc,
-                                     uint32_t id, int x, int y) {
-  if (!(x < s.W && y < s.H)) {
-    push_band(b, false, id, 0u, false);
-    return false;
-  }
-  const size_t idx = (size_t)y * s.W + x;
+__device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, const DevOut& out,
+                                     uint32_t id0, uint32_t x0, uint32_t y0) {
+  const int lane = lane_id();
+  const int x = (int)x0 + (lane & 7), y = (int)y0 + (lane >> 3);
+  const bool tile = out.rgb && out.hit && (int)x0 + 8 <= s.W && (int)y0 + 8 <= s.H;
+  uint32_t packed = 0;
+  const bool inside = x < s.W && y < s.H;
   RaySetup r;
-  setup_ray32<ESCAPE, SPH>(s, b.outs[sc], x, y, r);
-  const bool band = r.band && !r.degenerate;
-  if (!push_band(b, band, id, 0u, false) && band) return false;
-  const float phi0 = phi0_of(b.outs[sc], r);
-  MarchOut<float> mo;
-  bool sredo = false;
-  if (r.degenerate) {
-    degenerate_out(mo);
-  } else if (r.over) {
-    over_out(s, r, mo);
-  } else {
-    Lane<float> L;
-    const double du = (r.l - s.u0) * s.inv_nstep;
-    setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
-    if constexpr (SPH) setup_spheres32(s, r, L);
-    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(b.outs[sc]), mo);
-    if constexpr (SPH) sredo = L.sredo;
+  r.band = false;
+  if (inside) setup_ray32<ESCAPE, SPH>(s, out, x, y, r);
+  bool band = inside && r.band && !r.degenerate;
+  if (__any(band)) band = !push_band(b, band, id0 + (uint32_t)lane, 0u, false) && band;
+  const bool run = inside && !band;
+  bool redo = false;
+  uint32_t outcome = 0;
+  if (run) {
+    const size_t idx = (size_t)y * s.W + x;
+    const float phi0 = phi0_of(out, r);
+    MarchOut<float> mo;
+    bool sredo = false;
+    if (r.degenerate) {
+      degenerate_out(mo);
+    } else if (r.over) {
+      over_out(s, r, mo);
+    } else {
+      Lane<float> L;
+      const double du = (r.l - s.u0) * s.inv_nstep;
+      setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
+      if constexpr (SPH) setup_spheres32(s, r, L);
+      march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
+      if constexpr (SPH) sredo = L.sredo;
+    }
+    redo = finish_ray<ESCAPE>(s, out, idx, r, mo, phi0, tile, &packed) || sredo;
+    outcome = queue_outcome(mo.hit.cls, mo.steps);
   }
-  const bool redo = finish_ray<ESCAPE>(s, b.outs[sc], idx, r, mo, phi0) || sredo;
-  push_band(b, redo, id, queue_outcome(mo.hit.cls, mo.steps), true);
-  return true;
+  if (__any(redo)) push_band(b, redo, id0 + (uint32_t)lane_id(), outcome, true);
+  if (tile) store_tile(out, (uint32_t)s.W, x0, y0, packed);
+  return run;
 }
 
 template <bool ESCAPE, bool SPH>
 __device__ inline bool march_tile(const BatchDev& b, const DevScene& s, uint32_t sc,
-                                  uint32_t id) {
-  int x, y;
-  pixel_of(s, id - b.ray_off[sc], &x, &y);
-  return march_tile_xy<ESCAPE, SPH>(b, s, sc, id, x, y);
+                                  uint32_t id0) {
+  const DevOut out = b.outs[sc];
+  const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)((id0 - b.ray_off[sc]) >> 6));
+  const uint32_t ntx = ((uint32_t)s.W + 7) >> 3;
+  return march_tile_xy<ESCAPE, SPH>(b, s, out, id0, t % ntx * 8, t / ntx * 8);
 }
 
 // Tiles [b.tile_lo, b.tile_hi) hold scenes of one class (escape, spheres),
@@ -387,8 +434,7 @@ __device__ inline void run_tiles(const BatchDev& b, const DevScene* __restrict__
       const uint32_t id0 = (b.tile_lo + t) << 6;
       const uint32_t sc = (uint32_t)__builtin_amdgcn_readfirstlane((int)scene_of(b, id0));
       const DevScene& s = scenes[sc];
-      const uint32_t id = id0 + (uint32_t)lane_id();
-      const bool fin = march_tile<ESCAPE, SPH>(b, s, sc, id);
+      const bool fin = march_tile<ESCAPE, SPH>(b, s, sc, id0);
       note_finish(b, f, fin, sc);
     }
   }
@@ -399,7 +445,8 @@ __device__ inline void run_tiles(const BatchDev& b, const DevScene* __restrict__
 // wave's finish time goes to tile_end[tile] (reduced per scene afterwards).
 template <bool ESCAPE, bool SPH, int NS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8)))
-void batch_grid_kernel(BatchDev b, const DevScene* __restrict__ scenes) {
+void batch_grid_kernel(BatchDev b, const DevScene* __restrict__ scenes,
+                       const DevOut* __restrict__ outs, const uint2* __restrict__ info) {
   // the first workgroup is dispatched first: its start is the batch's
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicMin(b.t_start, (unsigned long long)wall_clock64());
@@ -407,10 +454,11 @@ void batch_grid_kernel(BatchDev b, const DevScene* __restrict__ scenes) {
   if (tile >= b.tile_hi) return;
   const uint32_t id0 = tile << 6;
   // the tile's scene and its position in the scene's grid of 8x8 tiles
-  const uint2 ti = b.tile_info[__builtin_amdgcn_readfirstlane((int)tile)];
-  const int lane = lane_id();
-  const int x = (int)(ti.y & 0xffffu) * 8 + (lane & 7), y = (int)(ti.y >> 16) * 8 + (lane >> 3);
-  march_tile_xy<ESCAPE, SPH, NS>(b, scenes[ti.x], ti.x, id0 + (uint32_t)lane, x, y);
+  // (restrict-qualified, so that these and the scene go to scalar registers)
+  const uint2 ti = info[__builtin_amdgcn_readfirstlane((int)tile)];
+  const DevOut out = outs[ti.x];
+  march_tile_xy<ESCAPE, SPH, NS>(b, scenes[ti.x], out, id0,
+                                 (ti.y & 0xffffu) * 8, (ti.y >> 16) * 8);
   if (lane_id() == 0) b.tile_end[tile] = (unsigned long long)wall_clock64();
 }
 
@@ -522,34 +570,34 @@ hipError_t launch_batch(const BatchDev& b, int cls, int block, int grid, hipStre
       case 0:
         if (ref)
           hipLaunchKernelGGL((batch_grid_kernel<false, false, kRefSteps>), g, dim3(block), 0,
-                             stream, b, b.scenes);
+                             stream, b, b.scenes, b.outs, b.tile_info);
         else
-          hipLaunchKernelGGL((batch_grid_kernel<false, false, 0>), g, dim3(block), 0, stream, b,
-                             b.scenes);
+          hipLaunchKernelGGL((batch_grid_kernel<false, false, 0>), g, dim3(block), 0,
+                             stream, b, b.scenes, b.outs, b.tile_info);
         break;
       case 1:
         if (ref)
           hipLaunchKernelGGL((batch_grid_kernel<true, false, kRefSteps>), g, dim3(block), 0,
-                             stream, b, b.scenes);
+                             stream, b, b.scenes, b.outs, b.tile_info);
         else
-          hipLaunchKernelGGL((batch_grid_kernel<true, false, 0>), g, dim3(block), 0, stream, b,
-                             b.scenes);
+          hipLaunchKernelGGL((batch_grid_kernel<true, false, 0>), g, dim3(block), 0,
+                             stream, b, b.scenes, b.outs, b.tile_info);
         break;
       case 2:
         if (ref)
           hipLaunchKernelGGL((batch_grid_kernel<false, true, kRefSteps>), g, dim3(block), 0,
-                             stream, b, b.scenes);
+                             stream, b, b.scenes, b.outs, b.tile_info);
         else
-          hipLaunchKernelGGL((batch_grid_kernel<false, true, 0>), g, dim3(block), 0, stream, b,
-                             b.scenes);
+          hipLaunchKernelGGL((batch_grid_kernel<false, true, 0>), g, dim3(block), 0,
+                             stream, b, b.scenes, b.outs, b.tile_info);
         break;
       default:
         if (ref)
           hipLaunchKernelGGL((batch_grid_kernel<true, true, kRefSteps>), g, dim3(block), 0,
-                             stream, b, b.scenes);
+                             stream, b, b.scenes, b.outs, b.tile_info);
         else
-          hipLaunchKernelGGL((batch_grid_kernel<true, true, 0>), g, dim3(block), 0, stream, b,
-                             b.scenes);
+          hipLaunchKernelGGL((batch_grid_kernel<true, true, 0>), g, dim3(block), 0,
+                             stream, b, b.scenes, b.outs, b.tile_info);
         break;
     }
     return hipGetLastError();

@@ -1056,12 +1056,14 @@ __device__ __forceinline__ void over_out(const DevScene& s, const RaySetup& r,
   mo.d = 0.f;
 }
 
-// Hit point, colour and output planes of one ray.  Returns true when the
-// ray's texel coordinate lies within the scene's edge guard of a texel edge:
-// its texel is then settled by the FP64 pass.
+// Hit point, colour and output planes of one ray; *packed = rgb | class << 24,
+// for the rgb and hit planes of a wave that stores them together (tile).
+// Returns true when the ray's texel coordinate lies within the scene's edge
+// guard of a texel edge: its texel is then settled by the FP64 pass.
 template <bool ESCAPE>
 __device__ inline bool finish_ray(const DevScene& s, const DevOut& out, size_t idx,
-                                  const RaySetup& r, const MarchOut<float>& mo, float phi0) {
+                                  const RaySetup& r, const MarchOut<float>& mo, float phi0,
+                                  bool tile = false, uint32_t* packed = nullptr) {
   const float e1x = r.sgn * s.e1f[0], e1y = r.sgn * s.e1f[1], e1z = r.sgn * s.e1f[2];
   uint32_t rgb = 0;
   bool redo = false;
@@ -1112,12 +1114,16 @@ __device__ inline bool finish_ray(const DevScene& s, const DevOut& out, size_t i
     const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
     rgb = equirect32(s.bg, dx * inv, dy * inv, dz * inv, s.edge_bg, &redo);
   }
-  if (out.rgb) {
-    out.rgb[3 * idx + 0] = (uint8_t)(rgb & 0xff);
-    out.rgb[3 * idx + 1] = (uint8_t)((rgb >> 8) & 0xff);
-    out.rgb[3 * idx + 2] = (uint8_t)((rgb >> 16) & 0xff);
+  if (tile) {
+    *packed = (rgb & 0xffffffu) | ((uint32_t)mo.hit.cls << 24);
+  } else {
+    if (out.rgb) {
+      out.rgb[3 * idx + 0] = (uint8_t)(rgb & 0xff);
+      out.rgb[3 * idx + 1] = (uint8_t)((rgb >> 8) & 0xff);
+      out.rgb[3 * idx + 2] = (uint8_t)((rgb >> 16) & 0xff);
+    }
+    if (out.hit) out.hit[idx] = (uint8_t)mo.hit.cls;
   }
-  if (out.hit) out.hit[idx] = (uint8_t)mo.hit.cls;
   if (out.steps) out.steps[idx] = mo.steps;
   if (out.hitpt) {
     out.hitpt[3 * idx + 0] = (double)qx;
