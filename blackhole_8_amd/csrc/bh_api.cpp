@@ -488,7 +488,10 @@ int check_tuning(bh_ctx* ctx, const bh_batch_tuning& t) {
 // Upload the plan and launch clear + persistent march + band pass (+ solo
 // scenes).  Events: ev0 before the march, ev1 after it, ev2 after the band
 // pass.  The tables go to the device with one synchronous copy each.
-int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bh::BatchDev* bd_out) {
+// times: the scenes' finish times are wanted (grid mode: a store a tile and a
+// reduction, 29 us over 1.2 million tiles).
+int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bool times,
+              bh::BatchDev* bd_out) {
   const size_t n = p.scenes.size();
   int rc;
   if ((rc = ensure(ctx, ctx->bscenes, n * sizeof(DevScene)))) return rc;
@@ -541,7 +544,7 @@ int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bh::Bat
   b.refill_steps = t.refill_steps;
   b.refill_idle = t.refill_idle;
   b.mode = t.mode;
-  b.tile_end = (unsigned long long*)ctx->btile.p;
+  b.tile_end = times ? (unsigned long long*)ctx->btile.p : nullptr;
   b.tile_info = t.mode == BH_BATCH_GRID ? (uint2*)ctx->btscene.p : nullptr;
   b.chunk = t.chunk;
   b.scene_end = (unsigned long long*)ctx->bend.p;
@@ -565,9 +568,15 @@ int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bh::Bat
       }
     }
   }
-  if (b.n_scenes > 0 && t.mode == BH_BATCH_GRID) HIP_TRY(ctx, bh::launch_batch_grid_finish(b, st));
+  if (b.n_scenes > 0 && t.mode == BH_BATCH_GRID && times)
+    HIP_TRY(ctx, bh::launch_batch_grid_finish(b, st));
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
-  if (b.n_scenes > 0) HIP_TRY(ctx, bh::launch_batch_band(b, st));
+  if (b.n_scenes > 0) {
+    int cls = -1;
+    for (int c = 0; c < 4; ++c)
+      if (p.cls_tile[c + 1] - p.cls_tile[c] == p.cls_tile[4]) cls = c;
+    HIP_TRY(ctx, bh::launch_batch_band(b, cls, st));
+  }
   // solo scenes: the per-frame kernels, with the context's band queue (the
   // band kernel clears it after each scene)
   if (!p.solo.empty()) {
@@ -1470,7 +1479,7 @@ int bh_render_batch_device(bh_ctx* ctx, int n, const bh_scene* scenes, const bh_
     if ((rc = plan_batch(ctx, n, scenes, options, outs, t.mode == BH_BATCH_LANES, &p))) return rc;
     (void)hipSetDevice(ctx->device);
     bh::BatchDev b;
-    if ((rc = run_batch(ctx, p, t, &b))) return rc;
+    if ((rc = run_batch(ctx, p, t, scene_ms != nullptr, &b))) return rc;
     if (!scene_ms && !stats) return BH_OK;
     HIP_TRY(ctx, hipEventSynchronize(ctx->ev2));
     if (stats) {
@@ -1534,7 +1543,7 @@ int bh_batch_autotune(bh_ctx* ctx, int n, const bh_scene* scenes, const bh_optio
       const BatchPlan& p = plans[m];
       double cms = 1e300;
       for (int r = 0; r < reps + 1; ++r) {  // first run warms up
-        if ((rc = run_batch(ctx, p, t, nullptr))) return rc;
+        if ((rc = run_batch(ctx, p, t, false, nullptr))) return rc;
         HIP_TRY(ctx, hipEventSynchronize(ctx->ev2));
         float ms = 0;
         HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev2));

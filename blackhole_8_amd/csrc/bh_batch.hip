@@ -325,54 +325,30 @@ __device__ inline void run_lanes(const BatchDev& b, uint32_t waves) {
   flush(b, f);
 }
 
-// The rgb and hit planes of a wave whose 64 lanes hold a whole tile of 8x8
-// pixels at (x0, y0), v = rgb | class << 24 on every lane: 48 lanes store a
-// dword of rgb and 16 a dword of classes, in one store instruction.  The
-// stores by lane (a short and two bytes of each pixel, eight rows of scenes of
-// any width) kept the texture-address unit busy for 290 cycles a wave, which
-// bounded a batch whose rays end early: 512 scenes, 77.6 Mpixel, took 930 us
-// in the grid launch and take 758.  (A frame's waves hold 16x4 pixels at
-// aligned rows and are bound by their arithmetic; packing cost them 8%.)
-__device__ __forceinline__ void store_tile(const DevOut& out, uint32_t W, uint32_t x0, uint32_t y0,
-                                           uint32_t v) {
-  const uint32_t t = (uint32_t)lane_id();
-  // classes of four neighbours in their first lane
-  const uint32_t v1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true);
-  const uint32_t h1 = __builtin_amdgcn_perm(v1, v, 0x0c0c0703u);
-  const uint32_t h2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h1, 0x4E, 0xf, 0xf, true);
-  const uint32_t h = __builtin_amdgcn_perm(h2, h1, 0x05040100u);
-  // dword j of a row holds bytes 4j .. 4j+3: from pixel j + j/3, byte j mod 3;
-  // lane 48 + 2 row + i holds the classes 4i .. 4i+3 of a row
-  const bool rgb = t < 48u;
-  const uint32_t row = rgb ? t * 43u >> 8 : (t - 48u) >> 1;
-  const uint32_t j = rgb ? t - 6u * row : t & 1u;
-  const uint32_t k = j < 3u ? j : j - 3u;
-  const uint32_t col = rgb ? (j < 3u ? j : j + 1u) : 4u * j;
-  const int src = (int)(4u * (8u * row + col));
-  const uint32_t a = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v);
-  const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute(src + 4, (int)v);
-  const uint32_t hh = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)h);
-  const uint32_t sel = k == 0u ? 0x04020100u : k == 1u ? 0x05040201u : 0x06050402u;
-  const uint32_t word = rgb ? __builtin_amdgcn_perm(b, a, sel) : hh;
-  const uint32_t pix = (y0 + row) * W + x0;
-  const uint64_t p = (rgb ? (uint64_t)out.rgb + 3ull * pix : (uint64_t)out.hit + pix) + 4u * j;
-  // planes of any alignment; device memory, also where the pointer was loaded
-  struct __attribute__((packed)) Word { uint32_t w; };
-  using GlobalWord = __attribute__((address_space(1))) Word;
-  reinterpret_cast<GlobalWord*>(p)->w = word;
+// The output record at a wave-uniform place, through the scalar cache, at this
+// point of the program.
+__device__ __forceinline__ DevOut load_out(const DevOut* p) {
+  uint64_t a = (uint64_t)p;
+  __asm__ volatile("" : "+s"(a));
+  using Const = __attribute__((address_space(4))) const uint64_t;
+  const Const* w = (const Const*)a;
+  return DevOut{(uint8_t*)w[0], (uint8_t*)w[1], (double*)w[2], (double*)w[3], (int32_t*)w[4]};
 }
+static_assert(sizeof(DevOut) == 40, "five pointers");
 
 // Tile mode: a wave takes a whole 8x8 tile of one scene and marches it with
 // the per-frame kernel's wave-uniform loop (scene constants in scalar
 // registers).  Returns whether this lane's ray was finished here (not queued
 // for the band pass).
 template <bool ESCAPE, bool SPH, int NS = 0>
-__device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, const DevOut& out,
-                                     uint32_t id0, uint32_t x0, uint32_t y0) {
+__device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s,
+                                     const DevOut* __restrict__ outp, uint32_t id0, uint32_t x0,
+                                     uint32_t y0) {
   const int lane = lane_id();
   const int x = (int)x0 + (lane & 7), y = (int)y0 + (lane >> 3);
-  const bool tile = out.rgb && out.hit && (int)x0 + 8 <= s.W && (int)y0 + 8 <= s.H;
-  uint32_t packed = 0;
+  // the record is read again after the march rather than kept in ten scalar
+  // registers through it, which cost a spilled one a lane write and read each
+  const DevOut out = *outp;
   const bool inside = x < s.W && y < s.H;
   RaySetup r;
   r.band = false;
@@ -399,21 +375,19 @@ __device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s, const
       march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
       if constexpr (SPH) sredo = L.sredo;
     }
-    redo = finish_ray<ESCAPE>(s, out, idx, r, mo, phi0, tile, &packed) || sredo;
+    redo = finish_ray<ESCAPE>(s, load_out(outp), idx, r, mo, phi0) || sredo;
     outcome = queue_outcome(mo.hit.cls, mo.steps);
   }
   if (__any(redo)) push_band(b, redo, id0 + (uint32_t)lane_id(), outcome, true);
-  if (tile) store_tile(out, (uint32_t)s.W, x0, y0, packed);
   return run;
 }
 
 template <bool ESCAPE, bool SPH>
 __device__ inline bool march_tile(const BatchDev& b, const DevScene& s, uint32_t sc,
                                   uint32_t id0) {
-  const DevOut out = b.outs[sc];
   const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)((id0 - b.ray_off[sc]) >> 6));
   const uint32_t ntx = ((uint32_t)s.W + 7) >> 3;
-  return march_tile_xy<ESCAPE, SPH>(b, s, out, id0, t % ntx * 8, t / ntx * 8);
+  return march_tile_xy<ESCAPE, SPH>(b, s, b.outs + sc, id0, t % ntx * 8, t / ntx * 8);
 }
 
 // Tiles [b.tile_lo, b.tile_hi) hold scenes of one class (escape, spheres),
@@ -444,7 +418,7 @@ __device__ inline void run_tiles(const BatchDev& b, const DevScene* __restrict__
 // Grid mode: one wave per tile of [b.tile_lo, b.tile_hi), no queue; the
 // wave's finish time goes to tile_end[tile] (reduced per scene afterwards).
 template <bool ESCAPE, bool SPH, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? (NS > 0 ? 6 : 1) : 8)))
 void batch_grid_kernel(BatchDev b, const DevScene* __restrict__ scenes,
                        const DevOut* __restrict__ outs, const uint2* __restrict__ info) {
   // the first workgroup is dispatched first: its start is the batch's
@@ -456,10 +430,9 @@ void batch_grid_kernel(BatchDev b, const DevScene* __restrict__ scenes,
   // the tile's scene and its position in the scene's grid of 8x8 tiles
   // (restrict-qualified, so that these and the scene go to scalar registers)
   const uint2 ti = info[__builtin_amdgcn_readfirstlane((int)tile)];
-  const DevOut out = outs[ti.x];
-  march_tile_xy<ESCAPE, SPH, NS>(b, scenes[ti.x], out, id0,
+  march_tile_xy<ESCAPE, SPH, NS>(b, scenes[ti.x], outs + ti.x, id0,
                                  (ti.y & 0xffffu) * 8, (ti.y >> 16) * 8);
-  if (lane_id() == 0) b.tile_end[tile] = (unsigned long long)wall_clock64();
+  if (b.tile_end && lane_id() == 0) b.tile_end[tile] = (unsigned long long)wall_clock64();
 }
 
 // Latest tile finish time of each scene (grid mode), and the earliest start.
@@ -493,68 +466,57 @@ __global__ __launch_bounds__(256) void batch_lane_kernel(BatchDev b) {
 }
 
 // FP64 pass over the queued rays (the per-frame FP64 pass's body with the
-// scene of each ray id): workgroup blk takes part blk / kQueueSubs of
-// sub-queue blk mod kQueueSubs.
+// scene of each ray id).  CLS: the class of all scenes (escape + 2 spheres),
+// or -1 where a batch mixes them: the instance of one class holds an FP64 ray
+// once, not four times (57 KB of code against 245).
+constexpr uint32_t kBatchEdgeParts = 32, kBatchBandWaves = 512;
+
+template <int CLS>
 __global__ __launch_bounds__(64) void batch_band_kernel(BatchDev b) {
-  const uint32_t k = blockIdx.x % kQueueSubs, part = blockIdx.x / kQueueSubs;
-  const uint32_t parts = gridDim.x / kQueueSubs;
-  const uint32_t nb = min(b.band.count[16 * k], b.band.sub_cap);
-  const uint32_t ne = min(b.band.count[16 * k + 2], b.band.sub_cap - nb);
-  const uint64_t* items = b.band.items + (size_t)k * b.band.sub_cap;
-  // band rays, then texel-edge rays (from the back)
-#pragma unroll 1
-  for (uint32_t i = part * blockDim.x + threadIdx.x; i < nb + ne; i += parts * blockDim.x) {
-    const uint64_t it = items[i < nb ? i : b.band.sub_cap - 1u - (i - nb)];
-    const uint32_t id = (uint32_t)it, outcome = (uint32_t)(it >> 32);
-    const uint32_t sc = scene_of(b, id);
-    const DevScene& s = b.scenes[sc];
-    int x, y;
-    pixel_of(s, id - b.ray_off[sc], &x, &y);
-    const size_t idx = (size_t)y * s.W + x;
-    const bool sph = s.n_spheres > 0;
-    if (s.escape) {
-      if (sph)
-        fp64_ray<true, true>(s, b.outs[sc], idx, x, y, outcome);
-      else
-        fp64_ray<true, false>(s, b.outs[sc], idx, x, y, outcome);
-    } else {
-      if (sph)
-        fp64_ray<false, true>(s, b.outs[sc], idx, x, y, outcome);
-      else
-        fp64_ray<false, false>(s, b.outs[sc], idx, x, y, outcome);
+  queue_rays(b.band, blockIdx.x, kBatchEdgeParts, kBatchBandWaves, []() {},
+             [&](uint32_t id, uint32_t outcome) {
+               const uint32_t sc = scene_of(b, id);
+               const DevScene& s = b.scenes[sc];
+               const DevOut& out = b.outs[sc];
+               int x, y;
+               pixel_of(s, id - b.ray_off[sc], &x, &y);
+               const size_t idx = (size_t)y * s.W + x;
+               const int cls = CLS >= 0 ? CLS : (s.escape ? 1 : 0) + (s.n_spheres > 0 ? 2 : 0);
+               if (cls == 0) fp64_ray<false, false>(s, out, idx, x, y, outcome);
+               if (cls == 1) fp64_ray<true, false>(s, out, idx, x, y, outcome);
+               if (cls == 2) fp64_ray<false, true>(s, out, idx, x, y, outcome);
+               if (cls == 3) fp64_ray<true, true>(s, out, idx, x, y, outcome);
+             });
+}
+
+// The launch's counters and queue counts cleared and, in grid mode, the scene
+// of every tile and the tile's column and row in the scene (workgroup s fills
+// scene s's tiles), so that a wave finds its scene and pixels with one load
+// rather than a search and a division.
+__global__ __launch_bounds__(256) void batch_clear_kernel(BatchDev b) {
+  const uint32_t s = blockIdx.x, t = threadIdx.x;
+  if (s == 0) {
+    if (t < 4) b.head[t] = 0u;
+    if (t < kQueueSubs) {
+      b.band.count[16 * t] = 0u;
+      b.band.count[16 * t + 2] = 0u;
     }
+    if (t == 0) b.t_start[0] = ~0ull;
   }
-}
-
-__global__ void batch_clear_kernel(BatchDev b) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < b.n_scenes) b.scene_end[i] = 0ull;
-  if (i < 4) b.head[i] = 0u;
-  if (i < kQueueSubs) {
-    b.band.count[16 * i] = 0u;
-    b.band.count[16 * i + 2] = 0u;
-  }
-  if (i == 0) b.t_start[0] = ~0ull;
-}
-
-// Grid mode: the scene of every tile and the tile's column and row in the
-// scene (workgroup s fills scene s's tiles), so that a wave finds its scene
-// and pixels with one load rather than a search and a division.
-__global__ __launch_bounds__(256) void batch_tile_info_kernel(BatchDev b) {
-  const uint32_t s = blockIdx.x;
+  if (s >= b.n_scenes) return;
+  if (t == 0) b.scene_end[s] = 0ull;
+  if (!b.tile_info) return;
   const uint32_t t0 = b.ray_off[s] >> 6, t1 = b.ray_off[s + 1] >> 6;
   const uint32_t ntx = ((uint32_t)b.scenes[s].W + 7) >> 3;
-  for (uint32_t t = t0 + threadIdx.x; t < t1; t += blockDim.x)
-    b.tile_info[t] = make_uint2(s, ((t - t0) % ntx) | (((t - t0) / ntx) << 16));
+  for (uint32_t i = t0 + t; i < t1; i += blockDim.x)
+    b.tile_info[i] = make_uint2(s, ((i - t0) % ntx) | (((i - t0) / ntx) << 16));
 }
 
 }  // namespace
 
 hipError_t launch_batch_clear(const BatchDev& b, hipStream_t stream) {
-  const uint32_t n = b.n_scenes > kQueueSubs ? b.n_scenes : kQueueSubs;
-  hipLaunchKernelGGL(batch_clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, b);
-  if (b.tile_info && b.n_scenes > 0)
-    hipLaunchKernelGGL(batch_tile_info_kernel, dim3(b.n_scenes), dim3(256), 0, stream, b);
+  hipLaunchKernelGGL(batch_clear_kernel, dim3(b.n_scenes ? b.n_scenes : 1), dim3(256), 0, stream,
+                     b);
   return hipGetLastError();
 }
 
@@ -632,9 +594,25 @@ hipError_t launch_batch_grid_finish(const BatchDev& b, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// 32 one-wave workgroups per sub-queue.
-hipError_t launch_batch_band(const BatchDev& b, hipStream_t stream) {
-  hipLaunchKernelGGL(batch_band_kernel, dim3(32 * kQueueSubs), dim3(64), 0, stream, b);
+hipError_t launch_batch_band(const BatchDev& b, int cls, hipStream_t stream) {
+  const dim3 g(kBatchEdgeParts * kQueueSubs + kBatchBandWaves), w(64);
+  switch (cls) {
+    case 0:
+      hipLaunchKernelGGL((batch_band_kernel<0>), g, w, 0, stream, b);
+      break;
+    case 1:
+      hipLaunchKernelGGL((batch_band_kernel<1>), g, w, 0, stream, b);
+      break;
+    case 2:
+      hipLaunchKernelGGL((batch_band_kernel<2>), g, w, 0, stream, b);
+      break;
+    case 3:
+      hipLaunchKernelGGL((batch_band_kernel<3>), g, w, 0, stream, b);
+      break;
+    default:
+      hipLaunchKernelGGL((batch_band_kernel<-1>), g, w, 0, stream, b);
+      break;
+  }
   return hipGetLastError();
 }
 

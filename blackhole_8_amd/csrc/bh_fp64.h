@@ -259,7 +259,9 @@ __device__ __forceinline__ int tex_index(double v, int n) {
 }
 
 __device__ __forceinline__ uint32_t texel(const DevTex& t, int col, int row) {
-  return t.data[(size_t)row * t.cols + col];
+  // (the record's pointer is a loaded one: say that it is device memory)
+  using Global = __attribute__((address_space(1))) const uint32_t;
+  return ((const Global*)(uintptr_t)t.data)[(size_t)row * t.cols + col];
 }
 
 // Bilinear sample at continuous texel coordinates (col a, row b), centres at

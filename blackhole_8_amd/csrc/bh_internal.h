@@ -209,7 +209,7 @@ struct BatchDev {
   int32_t refill_steps;      // steps between refill checks
   int32_t refill_idle;       // refill once at least this many lanes of 64 idle
   int32_t chunk;             // least tiles per queue pop
-  unsigned long long* tile_end;   // grid mode: finish time of each tile
+  unsigned long long* tile_end;   // grid mode: finish time of each tile (NULL: not asked)
   uint2* tile_info;               // grid mode: per tile its scene and (column | row << 16)
                                   // in the scene's tiles (set by the clear launch)
   unsigned long long* scene_end;  // per scene: latest finish time (wall clock)
@@ -218,7 +218,8 @@ struct BatchDev {
 
 // cls: scene class of a tile-mode launch, escape + 2 spheres
 hipError_t launch_batch(const BatchDev& b, int cls, int block, int grid, hipStream_t stream);
-hipError_t launch_batch_band(const BatchDev& b, hipStream_t stream);
+// cls: the class of all scenes, -1 where they differ
+hipError_t launch_batch_band(const BatchDev& b, int cls, hipStream_t stream);
 hipError_t launch_batch_grid_finish(const BatchDev& b, hipStream_t stream);
 hipError_t launch_batch_clear(const BatchDev& b, hipStream_t stream);
 

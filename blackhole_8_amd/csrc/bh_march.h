@@ -920,11 +920,11 @@ struct RaySetup {
   bool over;  // brief frames: the class is known without a march
 };
 
-// far2 (DevScene.far2; +inf: march every ray) and capt: an escaping ray with
-// b^2 > far2 meets nothing, and with capt the horizon class is all that is
-// asked of a captured one; such a ray ends here (r.over).
+// ends: an escaping ray with b^2 > far2 (DevScene.far2 or +inf) meets nothing,
+// and with capt the horizon class is all that is asked of a captured one; such
+// a ray ends here (r.over).
 __device__ inline void setup_ray(const DevScene& s, int x, int y, bool force_bisect,
-                                 RaySetup& r, double far2 = __builtin_inf(),
+                                 RaySetup& r, bool ends = false, double far2 = 0.0,
                                  bool capt = false) {
   // the pixel point pv = fvB - sx vy - sy vz (relative to B) enters only
   // through dv = F - pv (along yv), cv = pv x F (|cv| = b |dv|) and dv.F,
@@ -953,7 +953,8 @@ __device__ inline void setup_ray(const DevScene& s, int x, int y, bool force_bis
   r.e2x = r.e2y = r.e2z = 0.f;
   r.ib2 = 0.0;
   r.l = s.Uc;
-  r.over = !r.degenerate && !r.band && (r.captured ? capt : dF > 0.0 && cc > dd * far2);
+  r.over = ends && !r.degenerate && !r.band &&
+           (r.captured ? capt : dF > 0.0 && cc > dd * far2);
   if (r.degenerate || r.over) return;
   // 1 / b^2 = dd / cc: hardware reciprocal and two Newton steps (<= 2 ulp)
   double rc = __builtin_amdgcn_rcp(cc);
@@ -1038,7 +1039,7 @@ __device__ __forceinline__ void setup_ray32(const DevScene& s, const DevOut& out
     setup_ray(s, x, y, false, r);
   } else {
     const bool brief = brief_march(out);
-    setup_ray(s, x, y, false, r, brief ? s.far2 : __builtin_inf(),
+    setup_ray(s, x, y, false, r, true, brief ? s.far2 : __builtin_inf(),
               brief && !s.has_disc && !out.steps && !out.hitpt);
   }
 }
@@ -1056,14 +1057,17 @@ __device__ __forceinline__ void over_out(const DevScene& s, const RaySetup& r,
   mo.d = 0.f;
 }
 
-// Hit point, colour and output planes of one ray; *packed = rgb | class << 24,
-// for the rgb and hit planes of a wave that stores them together (tile).
-// Returns true when the ray's texel coordinate lies within the scene's edge
-// guard of a texel edge: its texel is then settled by the FP64 pass.
+template <typename T> using global_ptr = __attribute__((address_space(1))) T*;
+template <typename T> __device__ __forceinline__ global_ptr<T> to_global(T* p) {
+  return (global_ptr<T>)(uintptr_t)p;
+}
+
+// Hit point, colour and output planes of one ray.  Returns true when the
+// ray's texel coordinate lies within the scene's edge guard of a texel edge:
+// its texel is then settled by the FP64 pass.
 template <bool ESCAPE>
 __device__ inline bool finish_ray(const DevScene& s, const DevOut& out, size_t idx,
-                                  const RaySetup& r, const MarchOut<float>& mo, float phi0,
-                                  bool tile = false, uint32_t* packed = nullptr) {
+                                  const RaySetup& r, const MarchOut<float>& mo, float phi0) {
   const float e1x = r.sgn * s.e1f[0], e1y = r.sgn * s.e1f[1], e1z = r.sgn * s.e1f[2];
   uint32_t rgb = 0;
   bool redo = false;
@@ -1114,23 +1118,26 @@ __device__ inline bool finish_ray(const DevScene& s, const DevOut& out, size_t i
     const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
     rgb = equirect32(s.bg, dx * inv, dy * inv, dz * inv, s.edge_bg, &redo);
   }
-  if (tile) {
-    *packed = (rgb & 0xffffffu) | ((uint32_t)mo.hit.cls << 24);
-  } else {
-    if (out.rgb) {
-      out.rgb[3 * idx + 0] = (uint8_t)(rgb & 0xff);
-      out.rgb[3 * idx + 1] = (uint8_t)((rgb >> 8) & 0xff);
-      out.rgb[3 * idx + 2] = (uint8_t)((rgb >> 16) & 0xff);
-    }
-    if (out.hit) out.hit[idx] = (uint8_t)mo.hit.cls;
+  // (global stores, also where the record was loaded: flat ones of bytes and
+  // shorts took the address unit a lane at a time, 64% of a batch's grid
+  // launch; 512 scenes, 77.6 Mpixel, 930 us with them, 695 with these.
+  // Gathering a tile's planes across lanes into one dword store a lane took
+  // 758, its dwords being misaligned in scenes of odd widths.)
+  if (out.rgb) {
+    global_ptr<uint8_t> p = to_global(out.rgb) + 3 * idx;
+    p[0] = (uint8_t)(rgb & 0xff);
+    p[1] = (uint8_t)((rgb >> 8) & 0xff);
+    p[2] = (uint8_t)((rgb >> 16) & 0xff);
   }
-  if (out.steps) out.steps[idx] = mo.steps;
+  if (out.hit) to_global(out.hit)[idx] = (uint8_t)mo.hit.cls;
+  if (out.steps) to_global(out.steps)[idx] = mo.steps;
   if (out.hitpt) {
-    out.hitpt[3 * idx + 0] = (double)qx;
-    out.hitpt[3 * idx + 1] = (double)qy;
-    out.hitpt[3 * idx + 2] = (double)qz;
+    global_ptr<double> p = to_global(out.hitpt) + 3 * idx;
+    p[0] = (double)qx;
+    p[1] = (double)qy;
+    p[2] = (double)qz;
   }
-  if (out.phi) out.phi[idx] = r.degenerate ? mo.a : (double)phi0 + mo.a;
+  if (out.phi) to_global(out.phi)[idx] = r.degenerate ? mo.a : (double)phi0 + mo.a;
   return redo;
 }
 
@@ -1454,7 +1461,7 @@ __device__ inline void march64e(const DevScene& s, Lane<double>& L, bool capture
 // disagrees, and scenes with spheres (the event march tests spheres with an
 // FP32 table).
 template <bool ESCAPE, bool SPH>
-__device__ inline void fp64_ray(const DevScene& s, const DevOut& out, size_t idx, int x, int y,
+__device__ __forceinline__ void fp64_ray(const DevScene& s, const DevOut& out, size_t idx, int x, int y,
                                 uint32_t outcome) {
   Pixel64 px;
   RaySetup r;
@@ -1485,6 +1492,64 @@ __device__ inline void fp64_ray(const DevScene& s, const DevOut& out, size_t idx
   }
   trace64(s, x, y, px);
   store_pixel64(out, idx, px);
+}
+
+// FP64 pass over a queue, by one-wave workgroups of two kinds, so that no
+// wave mixes the band rays' full FP64 march with the texel-edge rays' short
+// refinement: workgroups blk < kQueueSubs * R take the texel-edge rays (the
+// back of the sub-queues; blk takes part blk / kQueueSubs of sub-queue blk mod
+// kQueueSubs), the nband workgroups after them the band rays of all sub-queues
+// packed together (the front segments, indexed through their prefix sum).
+// begin() runs in a wave that has rays, ray(id, outcome) for each of them; one
+// loop serves the rays of either kind, so that both run the same code (an FP64
+// ray inlined twice doubles what the instruction cache has to fetch).
+template <typename B, typename F>
+__device__ __forceinline__ void queue_rays(const DevQueue& q, uint32_t blk, uint32_t R,
+                                           uint32_t nband, B begin, F ray) {
+  __shared__ uint32_t pre[kQueueSubs + 1];
+  const uint32_t lane = threadIdx.x;
+  const bool edge = blk < kQueueSubs * R;
+  uint32_t first, stride, total, k = 0;
+  if (edge) {
+    k = blk % kQueueSubs;
+    const uint32_t nb = min(q.count[16 * k], q.sub_cap);
+    total = min(q.count[16 * k + 2], q.sub_cap - nb);
+    first = blk / kQueueSubs * 64;
+    stride = R * 64;
+  } else {
+    // pre[k] = band rays of sub-queues 0 .. k-1
+    uint32_t sum = min(q.count[16 * lane], q.sub_cap);
+#pragma unroll
+    for (int j = 1; j < 64; j <<= 1) {
+      const uint32_t v = __shfl_up(sum, j);
+      if (lane >= (uint32_t)j) sum += v;
+    }
+    if (lane == 0) pre[0] = 0;
+    pre[lane + 1] = sum;
+    __syncthreads();
+    total = pre[kQueueSubs];
+    first = (blk - kQueueSubs * R) * 64;
+    stride = nband * 64;
+  }
+  if (first < total) begin();
+#pragma unroll 1
+  for (uint32_t i = first + lane; i < total; i += stride) {
+    uint64_t it;
+    if (edge) {
+      it = q.items[(size_t)k * q.sub_cap + (q.sub_cap - 1u - i)];
+    } else {
+      uint32_t lo = 0, hi = kQueueSubs;  // the lo with pre[lo] <= i < pre[lo + 1]
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (pre[mid] <= i)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      it = (uint32_t)q.items[(size_t)lo * q.sub_cap + (i - pre[lo])];
+    }
+    ray((uint32_t)it, (uint32_t)(it >> 32));
+  }
 }
 
 }  // namespace bh

@@ -80,9 +80,11 @@ __device__ __forceinline__ void march_pixel(const DevScene& s, const DevOut& out
     queue_push_edge(q, k, (uint32_t)idx, queue_outcome(mo.hit.cls, mo.steps));
 }
 
-// Without spheres the march fits 64 VGPRs: 8 waves per SIMD.
+// Without spheres the march fits 64 VGPRs: 8 waves per SIMD; with them the
+// instance compiled for its step count fits 80, 6 waves (5 waves: 56 us a
+// 1280x720 frame of 16 spheres against 52).
 template <bool ESCAPE, bool SPH, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? (NS > 0 ? 6 : 1) : 8)))
 void march_kernel(const DevScene* __restrict__ sp, DevOut out, DevQueue q) {
   const DevScene& s = *sp;
   const int x = blockIdx.x * 16 + (threadIdx.x & 15);
@@ -108,7 +110,7 @@ __device__ __forceinline__ void frame_slice(const DevOut& out, const DevQueue& q
 // Every frame of a camera path in one launch (blockIdx.z = frame - frame0):
 // consecutive frames share no ramp-up or drain of the machine.
 template <bool ESCAPE, bool SPH, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? (NS > 0 ? 6 : 1) : 8)))
 void march_frames_kernel(const DevScene* __restrict__ sp, DevOut out, DevQueue q, size_t npix,
                          int frame0) {
   const int f = frame0 + (int)blockIdx.z;
@@ -122,13 +124,6 @@ void march_frames_kernel(const DevScene* __restrict__ sp, DevOut out, DevQueue q
   march_pixel<ESCAPE, SPH, NS>(s, o, qf, queue_sub(blockIdx.x, blockIdx.y), x, y);
 }
 
-// FP64 pass over one frame's queue, by one-wave workgroups of two kinds, so
-// that no wave mixes the band rays' full FP64 march with the texel-edge rays'
-// short refinement: workgroups blk < kQueueSubs * R take the texel-edge rays
-// (the back of the sub-queues; blk takes part blk / kQueueSubs of sub-queue
-// blk mod kQueueSubs), the nband workgroups after them the band rays of all
-// sub-queues packed together (the front segments, indexed through their
-// prefix sum).
 // One round of vector loads over the scene record's 64-byte lines, a lane
 // each, before a wave's first ray: a wave of this pass runs nearly alone on
 // its CU after the march has filled L2 with framebuffer lines, so the scalar
@@ -142,57 +137,15 @@ __device__ __forceinline__ void touch_scene(const DevScene& s, uint32_t lane) {
   }
 }
 
+// The queued rays of one frame.
 template <bool ESCAPE, bool SPH>
 __device__ __forceinline__ void band_rays(const DevScene& s, const DevOut& out, const DevQueue& q,
                                           uint32_t blk, uint32_t R, uint32_t nband) {
-  __shared__ uint32_t pre[kQueueSubs + 1];
-  const uint32_t lane = threadIdx.x;
-  // one loop over the rays of either kind, so that both run the same code (an
-  // FP64 ray inlined twice doubles what the instruction cache has to fetch)
-  const bool edge = blk < kQueueSubs * R;
-  uint32_t first, stride, total, k = 0;
-  if (edge) {
-    k = blk % kQueueSubs;
-    const uint32_t nb = min(q.count[16 * k], q.sub_cap);
-    total = min(q.count[16 * k + 2], q.sub_cap - nb);
-    first = blk / kQueueSubs * 64;
-    stride = R * 64;
-  } else {
-    // pre[k] = band rays of sub-queues 0 .. k-1
-    uint32_t sum = min(q.count[16 * lane], q.sub_cap);
-#pragma unroll
-    for (int j = 1; j < 64; j <<= 1) {
-      const uint32_t v = __shfl_up(sum, j);
-      if (lane >= (uint32_t)j) sum += v;
-    }
-    if (lane == 0) pre[0] = 0;
-    pre[lane + 1] = sum;
-    __syncthreads();
-    total = pre[kQueueSubs];
-    first = (blk - kQueueSubs * R) * 64;
-    stride = nband * 64;
-  }
-  if (first < total) touch_scene(s, lane);
-#pragma unroll 1
-  for (uint32_t i = first + lane; i < total; i += stride) {
-    uint64_t it;
-    if (edge) {
-      it = q.items[(size_t)k * q.sub_cap + (q.sub_cap - 1u - i)];
-    } else {
-      uint32_t lo = 0, hi = kQueueSubs;  // the lo with pre[lo] <= i < pre[lo + 1]
-      while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (pre[mid] <= i)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      it = (uint32_t)q.items[(size_t)lo * q.sub_cap + (i - pre[lo])];
-    }
-    const uint32_t idx = (uint32_t)it;
-    fp64_ray<ESCAPE, SPH>(s, out, idx, (int)(idx % (uint32_t)s.W), (int)(idx / (uint32_t)s.W),
-                          (uint32_t)(it >> 32));
-  }
+  queue_rays(q, blk, R, nband, [&]() { touch_scene(s, threadIdx.x); },
+             [&](uint32_t idx, uint32_t outcome) {
+               fp64_ray<ESCAPE, SPH>(s, out, idx, (int)(idx % (uint32_t)s.W),
+                                     (int)(idx / (uint32_t)s.W), outcome);
+             });
 }
 
 // Workgroups of the FP64 pass of one frame: edge workgroups per sub-queue and
