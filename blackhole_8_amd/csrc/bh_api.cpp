@@ -300,8 +300,15 @@ int build_scene(bh_ctx* ctx, const bh_scene* sc, const bh_options* opt_in, DevSc
   // comes nearer than r_t (1 - d^2/8).  b^2 >= 1.6 b_c^2 puts r_t beyond
   // 5.1M (1 - 3M/r_t >= 0.41), which clears the horizon from 5 steps on.
   d->reach = d->has_disc && d->r_out >= 0.0 ? (float)(d->r_out * (1.0 + 1e-4)) : 0.f;
+  // (Only where the ray's l lies in its bracket, the points' rounding is far
+  // below the margins, and the disc is centred on the hole.)
   d->far2 = std::numeric_limits<double>::infinity();
-  if (d->nstep >= 5) {
+  const double absB = std::sqrt(d->B[0] * d->B[0] + d->B[1] * d->B[1] + d->B[2] * d->B[2]);
+  const double n2 = d->dn[0] * d->dn[0] + d->dn[1] * d->dn[1] + d->dn[2] * d->dn[2];
+  const bool centred = !d->has_disc || (d->dv0[0] == d->B[0] && d->dv0[1] == d->B[1] &&
+                                        d->dv0[2] == d->B[2] && n2 < 1e30 && d->r_out < 1e150);
+  if (d->nstep >= 5 && !d->escape && d->n_spheres == 0 && centred && absB < 1e5 * d->M &&
+      d->u0 < d->Uc && d->u0 > d->l0) {
     d->far2 = 1.6 * d->bc2;
     const double R = d->reach;
     if (R > 0.0) {

@@ -55,3 +55,22 @@ def test_brief_planes_equal_the_full_march(renderer, nstep, disc):
             got = renderer.render(s, o, want)
             for k in want:
                 assert got[k].tobytes() == full[k].tobytes(), (k, dist)
+
+
+@pytest.mark.parametrize("scale", [1e-3, 1e4, 1e6])
+@pytest.mark.parametrize("disc", [None, (12.0, 3.0)])
+def test_brief_planes_at_other_scales(renderer, scale, disc):
+    """Lengths at which the turning point leaves its solver's bracket too."""
+    rng = np.random.default_rng(7)
+    renderer.set_textures(scenes.disc_orbit(W, H).textures)
+    for dist in (6.5, 20.0, 48.0):
+        s = _scene(rng, dist * scale, None if disc is None else (disc[0] * scale, disc[1] * scale),
+                   (0.0, 0.0, 0.0))
+        s.hole.mass *= scale
+        o = scenes.options(precision=abi.PREC_FP32)
+        print(f"[case] brief march at scale {scale} disc {disc} from {dist}", flush=True)
+        full = renderer.render(s, o, ("rgb", "hit", "steps", "hitpt", "phi"))
+        for want in (("rgb", "hit", "steps", "hitpt"), ("rgb", "hit")):
+            got = renderer.render(s, o, want)
+            for k in want:
+                assert got[k].tobytes() == full[k].tobytes(), (k, dist)
