@@ -1594,10 +1594,9 @@ static int build_flat(bh_ctx* ctx, const bh_flat_scene* sc, bh::DevFlat* dp) {
   d.n_planes = sc->n_planes;
   d.steps = sc->steps;
   for (int i = 0; i < sc->n_rects; ++i) {
-    for (int v = 0; v < 5; ++v) {
+    for (int v = 0; v < 5; ++v)
       if (!finite3(sc->rects[i].vertex[v])) return fail(ctx, BH_ERR_INVALID_ARG, "rectangle vertices must be finite");
-      copy3(d.rv[i][v], sc->rects[i].vertex[v]);
-    }
+    bh::flat_rect(&d.rect[i], sc->rects[i].vertex);
     d.rtex[i] = devtex(ctx, sc->rects[i].texture);
     if (!d.rtex[i].data)
       return fail(ctx, BH_ERR_EMPTY_TEXTURE, "rectangle texture slot is empty (Material::SetTexture)");
@@ -1612,11 +1611,11 @@ static int build_flat(bh_ctx* ctx, const bh_flat_scene* sc, bh::DevFlat* dp) {
         !(p.pattern_size >= 1.0 && p.pattern_size <= 536870912.0 &&
           p.pattern_size == std::floor(p.pattern_size)))
       return fail(ctx, BH_ERR_INVALID_ARG, "plane pattern_size must be 0 or a whole number in 1..2^29");
-    copy3(d.pp[i], p.position);
-    copy3(d.px[i], p.axis_x);
-    copy3(d.py[i], p.axis_y);
-    copy3(d.pz[i], p.axis_z);
-    d.psize[i] = p.pattern_size;
+    copy3(d.plane[i].p, p.position);
+    copy3(d.plane[i].x, p.axis_x);
+    copy3(d.plane[i].y, p.axis_y);
+    copy3(d.plane[i].z, p.axis_z);
+    d.plane[i].size = p.pattern_size;
   }
   return BH_OK;
 }

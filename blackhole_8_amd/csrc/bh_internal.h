@@ -227,16 +227,24 @@ hipError_t launch_batch_clear(const BatchDev& b, hipStream_t stream);
 // Flat-space scene (RayTracer::Prograde, ray_tracer.h:52-96): straight chords,
 // rectangles and chess-patterned infinite planes.  Passed by value.
 // ---------------------------------------------------------------------------
+struct DevRect {
+  double n[3], p[3];   // unit normal, vertex p1
+  double e1[3], e3[3]; // edges to p2 and p4
+  double d1, d3, l1, l3;  // their squared lengths and lengths
+};
+struct DevPlane {
+  double z[3], p[3], x[3], y[3], size;
+};
 struct DevFlat {
   double C[3], fv[3], vy[3], vz[3];  // camera position, focus vector, axes y, z
   int32_t W, H, n_rects, n_planes, steps, pad0;
-  double rv[BH_MAX_RECTS][5][3];     // rectangle vertices ([0] pivot, [1..4] p1..p4)
+  DevRect rect[BH_MAX_RECTS];
+  DevPlane plane[BH_MAX_PLANES];
   DevTex rtex[BH_MAX_RECTS];
-  double pp[BH_MAX_PLANES][3], px[BH_MAX_PLANES][3], py[BH_MAX_PLANES][3],
-      pz[BH_MAX_PLANES][3];
-  double psize[BH_MAX_PLANES];
 };
 
+// A rectangle from its vertices ([0] pivot, [1..4] p1..p4).
+void flat_rect(DevRect* r, const double (*v)[3]);
 hipError_t launch_flat(const DevFlat& s, const DevOut& out, hipStream_t stream);
 
 // ---------------------------------------------------------------------------
