@@ -554,6 +554,12 @@ int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bool ti
   b.tile_end = times ? (unsigned long long*)ctx->btile.p : nullptr;
   b.tile_info = t.mode == BH_BATCH_GRID ? (uint2*)ctx->btscene.p : nullptr;
   b.chunk = t.chunk;
+  // runs of up to four tiles a wave, while each of the machine's wave slots
+  // still gets 16 runs to balance (512 scenes, 1.2 million tiles: 795 us with
+  // one tile, 750 with two or four, 773 with eight; without discs 543, 452 and
+  // 430, 433)
+  const uint32_t slots = (uint32_t)std::max(1, ctx->n_cu) * 32u;
+  b.tile_run = (int32_t)std::min<uint32_t>(4u, std::max<uint32_t>(1u, n_tiles / (16u * slots)));
   b.scene_end = (unsigned long long*)ctx->bend.p;
   HIP_TRY(ctx, bh::launch_batch_clear(b, st));
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));

@@ -209,6 +209,7 @@ struct BatchDev {
   int32_t refill_steps;      // steps between refill checks
   int32_t refill_idle;       // refill once at least this many lanes of 64 idle
   int32_t chunk;             // least tiles per queue pop
+  int32_t tile_run;          // grid mode: consecutive tiles of a wave
   unsigned long long* tile_end;   // grid mode: finish time of each tile (NULL: not asked)
   uint2* tile_info;               // grid mode: per tile its scene and (column | row << 16)
                                   // in the scene's tiles (set by the clear launch)
