@@ -183,12 +183,20 @@ __global__ void zero_u32_kernel(uint32_t* p, int n) {
 // Scene record and queue counts of a frame in place.  A kernel rather than
 // hipMemcpyAsync / hipMemsetAsync, so the call may also be captured in a
 // graph.
-__global__ __launch_bounds__(256) void scene_kernel(DevScene s, DevScene* dst, uint32_t* count) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
-  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-  for (uint32_t i = threadIdx.x; i < sizeof(DevScene) / 4; i += 256) d[i] = src[i];
+// One load a thread, not a loop of loads each waited for: bound by the
+// latency of the argument's loads (a 320x180 FP64 frame 34.4 -> 33.1 us, a
+// 1920x1080 FP32 one 46.0 -> 45.5).
+constexpr uint32_t kSceneThreads = 384;
+static_assert(sizeof(DevScene) % 8 == 0 && sizeof(DevScene) <= 8 * kSceneThreads,
+              "a double word a thread");
+__global__ __launch_bounds__(kSceneThreads) void scene_kernel(DevScene s, DevScene* dst,
+                                                              uint32_t* count) {
+  const uint32_t t = threadIdx.x;
+  uint64_t v = 0;
+  if (t < sizeof(DevScene) / 8) v = reinterpret_cast<const uint64_t*>(&s)[t];
   if (count)
-    for (uint32_t i = threadIdx.x; i < kQueueCountWords; i += 256) count[i] = 0u;
+    for (uint32_t i = t; i < kQueueCountWords; i += kSceneThreads) count[i] = 0u;
+  if (t < sizeof(DevScene) / 8) reinterpret_cast<uint64_t*>(dst)[t] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -345,7 +353,7 @@ hipError_t launch_scene(const DevScene& s, DevScene* dst, uint32_t* count, hipSt
   static_assert(sizeof(DevScene) % 4 == 0, "scene record is copied as 32-bit words");
   static_assert(sizeof(DevScene) + 2 * sizeof(void*) <= 4096,
                 "the scene record is passed as a kernel argument");
-  hipLaunchKernelGGL(scene_kernel, dim3(1), dim3(256), 0, stream, s, dst, count);
+  hipLaunchKernelGGL(scene_kernel, dim3(1), dim3(kSceneThreads), 0, stream, s, dst, count);
   return hipGetLastError();
 }
 
