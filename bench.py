@@ -391,6 +391,8 @@ def main() -> int:
         "band_launch_ms": round(band_ms, 4),
         "single_frame_kernel_ms": round(sum(m for m, _, _ in single) / len(single), 5),
         "flop_per_frame": round(work / F),
+        "flop_basis": "steps of the reference rule, also of rays whose march ends early "
+                      "because nothing is left for them to meet",
         "band_rays_per_frame": round(sum(n for _, _, n in single) / len(single), 1),
     }
 
