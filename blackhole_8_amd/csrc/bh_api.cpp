@@ -36,9 +36,9 @@ struct DevBuf {
 
 struct bh_ctx {
   int device = 0;
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr;  // the context's calls: own, or a caller's
+  hipStream_t own = nullptr;
   hipStream_t side = nullptr;  // band kernels of captured paths
-  bool own_stream = false;
   std::string err;
   DeviceTexture tex[BH_MAX_TEXTURES];
   DevBuf scene, rgb, hit, phi, hitpt, steps, qitems, qcount;
@@ -48,7 +48,11 @@ struct bh_ctx {
   int wall_khz = 0;
   void* noalloc = nullptr;  // this device's allocation-free scratch array
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
-  hipEvent_t ev_order = nullptr;  // orders a caller's stream after the context's
+  hipEvent_t ev_order = nullptr;  // orders one stream's work after another's
+  bool work = false;  // calls have put work on `stream` that no other stream follows
+  // tail: the context's last work is on another stream, tail_stream
+  hipStream_t tail_stream = nullptr;
+  bool tail = false;
   bool other_streams = false;  // a call has put work on a caller's stream
   char name[256] = {0};
   int n_cu = 0, clock_khz = 0;
@@ -132,6 +136,46 @@ int ensure(bh_ctx* ctx, DevBuf& b, size_t bytes) {
   if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
   b.bytes = bytes;
   return BH_OK;
+}
+
+// ---- order of the context's calls -------------------------------------------
+// A context's calls share its scene record, queues, tables and textures, so they
+// follow each other in the order they were made, whatever streams they run on: a
+// call whose stream differs from the last one's has it wait for that by event.
+// (Nothing is recorded after a call: that took a 512x512 image on a caller's
+// stream from 19.8 to 22.8 us.  A capture cannot wait for work outside it, so a
+// captured call's order is the caller's.)
+
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// st waits for what `before` holds.
+void follow(bh_ctx* ctx, hipStream_t st, hipStream_t before) {
+  if (hipStreamQuery(before) == hipSuccess) return;
+  (void)hipGetLastError();
+  if (hipEventRecord(ctx->ev_order, before) != hipSuccess ||
+      hipStreamWaitEvent(st, ctx->ev_order, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipDeviceSynchronize();
+  }
+}
+
+// st waits for the tail, if there is one.
+void follow_tail(bh_ctx* ctx, hipStream_t st) {
+  if (!ctx->tail || ctx->tail_stream == st || capturing(st) || capturing(ctx->tail_stream)) return;
+  follow(ctx, st, ctx->tail_stream);
+  ctx->tail = false;
+}
+
+// The context's stream, for a call about to put work on it.
+hipStream_t work_stream(bh_ctx* ctx) {
+  follow_tail(ctx, ctx->stream);
+  ctx->work = true;
+  return ctx->stream;
 }
 
 bool finite3(const double* v) {
@@ -516,7 +560,7 @@ int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bool ti
   const uint32_t sub_cap = std::max<uint32_t>((n_tiles + bh::kQueueSubs - 1) / bh::kQueueSubs, 1u) * 64u;
   if ((rc = ensure(ctx, ctx->bband, (size_t)sub_cap * bh::kQueueSubs * sizeof(uint64_t)))) return rc;
   if ((rc = ensure(ctx, ctx->bbandc, bh::kQueueCountWords * sizeof(uint32_t)))) return rc;
-  hipStream_t st = ctx->stream;
+  hipStream_t st = work_stream(ctx);
   // the persistent march reads the FP32 scenes by position in the plan
   std::vector<DevScene> fs;
   std::vector<DevOut> fo;
@@ -715,24 +759,19 @@ size_t diff_work(int W, int H) {
   return (size_t)bh::diff_partial_blocks(W, H) * 5 * sizeof(double);
 }
 
-// Readies the context for a call on a stream of the caller's: the stream waits
-// for what the context's own stream still holds.  (A capture cannot wait for
-// work outside it.)
+// Readies a stream of the caller's for a call.
 void enter_stream(bh_ctx* ctx, hipStream_t st) {
-  if (st == ctx->stream) return;
-  ctx->other_streams = true;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
+  if (st == ctx->stream) {
+    (void)work_stream(ctx);
     return;
   }
-  if (hipStreamQuery(ctx->stream) == hipSuccess) return;
-  (void)hipGetLastError();
-  if (hipEventRecord(ctx->ev_order, ctx->stream) != hipSuccess ||
-      hipStreamWaitEvent(st, ctx->ev_order, 0) != hipSuccess) {
-    (void)hipGetLastError();
-    (void)hipStreamSynchronize(ctx->stream);
-  }
+  ctx->other_streams = true;
+  if (capturing(st)) return;
+  follow_tail(ctx, st);
+  if (ctx->work) follow(ctx, st, ctx->stream);
+  ctx->work = false;
+  ctx->tail_stream = st;
+  ctx->tail = true;
 }
 
 // Waits for all work the context's calls have put on the device.
@@ -815,15 +854,15 @@ int bh_ctx_create(int device, bh_ctx** out) {
     if (e != hipSuccess) return fail(nullptr, BH_ERR_HIP, "hipSetDevice failed");
     bh_ctx* c = new bh_ctx();
     c->device = device;
-    e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
+    e = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking);
     if (e != hipSuccess) {
       delete c;
       return fail(nullptr, BH_ERR_HIP, "hipStreamCreate failed");
     }
-    c->own_stream = true;
+    c->stream = c->own;
     e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
     if (e != hipSuccess) {
-      (void)hipStreamDestroy(c->stream);
+      (void)hipStreamDestroy(c->own);
       delete c;
       return fail(nullptr, BH_ERR_HIP, "hipStreamCreate failed");
     }
@@ -862,7 +901,7 @@ void bh_ctx_destroy(bh_ctx* ctx) {
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev2) (void)hipEventDestroy(ctx->ev2);
   if (ctx->ev_order) (void)hipEventDestroy(ctx->ev_order);
-  if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
+  if (ctx->own) (void)hipStreamDestroy(ctx->own);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   delete ctx;
 }
@@ -886,18 +925,16 @@ int bh_ctx_set_stream(bh_ctx* ctx, void* stream) {
   return guarded(ctx, [&]() -> int {
     if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
     (void)hipSetDevice(ctx->device);
-    if (ctx->own_stream && ctx->stream) {
-      (void)hipStreamSynchronize(ctx->stream);
-      (void)hipStreamDestroy(ctx->stream);
+    const hipStream_t st = stream ? (hipStream_t)stream : ctx->own;
+    if (ctx->stream == ctx->own) {
+      (void)hipStreamSynchronize(ctx->own);
+      ctx->work = false;
+    } else if (ctx->stream != st && ctx->work) {
+      ctx->tail_stream = ctx->stream;
+      ctx->tail = ctx->other_streams = true;
+      ctx->work = false;
     }
-    if (stream) {
-      ctx->stream = (hipStream_t)stream;
-      ctx->own_stream = false;
-    } else {
-      hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
-      if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamCreate");
-      ctx->own_stream = true;
-    }
+    ctx->stream = st;
     return BH_OK;
   });
 }
@@ -980,7 +1017,7 @@ int bh_render_device(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
     if ((rc = queue_buffers(ctx, d.W, d.H, &q))) return rc;
     DevOut o{out_device->rgb, out_device->hit, out_device->phi_end, out_device->hit_point,
              out_device->steps};
-    return launch_frame(ctx, d, (DevScene*)ctx->scene.p, o, q, ctx->stream);
+    return launch_frame(ctx, d, (DevScene*)ctx->scene.p, o, q, work_stream(ctx));
   });
 }
 
@@ -1004,7 +1041,7 @@ int bh_render_device_noalloc(bh_ctx* ctx, const bh_scene* scene, const bh_option
     DevOut o{out_device->rgb, out_device->hit, out_device->phi_end, out_device->hit_point,
              out_device->steps};
     const DevQueue q{l.items, l.count, bh::queue_sub_cap(d.W, d.H)};
-    return launch_frame(ctx, d, l.scene, o, q, ctx->stream);
+    return launch_frame(ctx, d, l.scene, o, q, work_stream(ctx));
   });
 }
 
@@ -1025,7 +1062,7 @@ int bh_render(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt, const b
     if (out->steps) { if ((rc = ensure(ctx, ctx->steps, npix * 4))) return rc; o.steps = (int32_t*)ctx->steps.p; }
     bh_outputs dev{o.rgb, o.hit, o.phi, o.hitpt, o.steps};
     if ((rc = bh_render_device(ctx, scene, opt, &dev))) return rc;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     if (out->rgb) HIP_TRY(ctx, hipMemcpyAsync(out->rgb, o.rgb, npix * 3, hipMemcpyDeviceToHost, st));
     if (out->hit) HIP_TRY(ctx, hipMemcpyAsync(out->hit, o.hit, npix, hipMemcpyDeviceToHost, st));
     if (out->phi_end) HIP_TRY(ctx, hipMemcpyAsync(out->phi_end, o.phi, npix * 8, hipMemcpyDeviceToHost, st));
@@ -1051,7 +1088,7 @@ int bh_time_render(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt, in
     if ((rc = ensure(ctx, ctx->scene, sizeof(DevScene)))) return rc;
     DevQueue q;
     if ((rc = queue_buffers(ctx, d.W, d.H, &q))) return rc;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     DevOut o{(uint8_t*)ctx->rgb.p, (uint8_t*)ctx->hit.p, nullptr, nullptr, nullptr};
     DevScene* ds = (DevScene*)ctx->scene.p;
     const bool fast = fp32_eligible(d);
@@ -1218,7 +1255,7 @@ int bh_path_launch(bh_path* p, float* ms) {
     if (!p) return fail(nullptr, BH_ERR_BAD_HANDLE, "path is NULL");
     bh_ctx* ctx = p->ctx;
     (void)hipSetDevice(ctx->device);
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     if (p->exec_band) {
       // the march graph, then the FP64 pass's, with timing events around each
       HIP_TRY(ctx, path_clear(p, st));
@@ -1264,8 +1301,9 @@ int bh_fma_issue_rate(bh_ctx* ctx, double* fp32_tflops, double* fp64_tflops) {
     int rc = ensure(ctx, ctx->probe, 256 * sizeof(double));
     if (rc) return rc;
     const int n_cu = ctx->n_cu > 0 ? ctx->n_cu : 1;
-    HIP_TRY(ctx, bh::fma_probe<float>(n_cu, ctx->stream, (float*)ctx->probe.p, fp32_tflops));
-    HIP_TRY(ctx, bh::fma_probe<double>(n_cu, ctx->stream, (double*)ctx->probe.p, fp64_tflops));
+    hipStream_t st = work_stream(ctx);
+    HIP_TRY(ctx, bh::fma_probe<float>(n_cu, st, (float*)ctx->probe.p, fp32_tflops));
+    HIP_TRY(ctx, bh::fma_probe<double>(n_cu, st, (double*)ctx->probe.p, fp64_tflops));
     return BH_OK;
   });
 }
@@ -1280,7 +1318,7 @@ int bh_chord_sincos(bh_ctx* ctx, const float* x_host, float* sc_host, int64_t n)
     if (rc) return rc;
     float* x = (float*)ctx->probe.p;
     float* out = x + n;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     HIP_TRY(ctx, hipMemcpyAsync(x, x_host, (size_t)n * sizeof(float), hipMemcpyHostToDevice, st));
     HIP_TRY(ctx, bh::launch_chord_sincos(x, out, (int)n, st));
     HIP_TRY(ctx, hipMemcpyAsync(sc_host, out, (size_t)n * 2 * sizeof(float),
@@ -1302,7 +1340,7 @@ int bh_turning_points(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
     const size_t npix = (size_t)d.W * d.H;
     if ((rc = ensure(ctx, ctx->scene, sizeof(DevScene)))) return rc;
     if ((rc = ensure(ctx, ctx->probe, npix * sizeof(double)))) return rc;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     HIP_TRY(ctx, hipMemcpyAsync(ctx->scene.p, &d, sizeof d, hipMemcpyHostToDevice, st));
     HIP_TRY(ctx, bh::launch_turning((const DevScene*)ctx->scene.p, (double*)ctx->probe.p, d.W,
                                     d.H, st));
@@ -1320,7 +1358,7 @@ int bh_path_time(bh_path* p, int iters, double* march_ms, double* band_ms) {
     if (!p->fused) return fail(ctx, BH_ERR_UNSUPPORTED, "path frames are not all in the FP32 march");
     if (iters <= 0) return fail(ctx, BH_ERR_INVALID_ARG, "iters must be positive");
     (void)hipSetDevice(ctx->device);
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     double tm = 0, tb = 0;
     for (int it = 0; it < iters; ++it) {
       HIP_TRY(ctx, path_clear(p, st));
@@ -1406,7 +1444,7 @@ int bh_diff_adjoint_device(bh_ctx* ctx, const bh_diff_params* p, int precision,
     if ((rc = ensure(ctx, ctx->dpart, diff_work(d.W, d.H)))) return rc;
     HIP_TRY(ctx, bh::launch_diff_adjoint(d, precision == BH_PREC_FP64, grad_rgb, rgb_out, hit_out,
                                          (double*)ctx->dpart.p, grad_out, overflow_out,
-                                         ctx->stream));
+                                         work_stream(ctx)));
     return BH_OK;
   });
 }
@@ -1451,7 +1489,7 @@ int bh_diff_time(bh_ctx* ctx, const bh_diff_params* p, int precision, int iters,
     if ((rc = ensure(ctx, ctx->drgb, npix * 3 * sizeof(float)))) return rc;
     if ((rc = ensure(ctx, ctx->dhit, npix))) return rc;
     if ((rc = ensure(ctx, ctx->dgin, npix * 3 * sizeof(float)))) return rc;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     // dL/drgb: every byte 0x3c, i.e. 0.0115 per channel
     HIP_TRY(ctx, hipMemsetAsync(ctx->dgin.p, 0x3c, npix * 3 * sizeof(float), st));
     float* rgb = (float*)ctx->drgb.p;
@@ -1635,7 +1673,7 @@ int bh_render_flat_device(bh_ctx* ctx, const bh_flat_scene* sc, const bh_outputs
     if (rc) return rc;
     (void)hipSetDevice(ctx->device);
     DevOut o{out->rgb, out->hit, out->phi_end, out->hit_point, out->steps};
-    HIP_TRY(ctx, bh::launch_flat(d, o, ctx->stream));
+    HIP_TRY(ctx, bh::launch_flat(d, o, work_stream(ctx)));
     return BH_OK;
   });
 }
@@ -1655,7 +1693,7 @@ int bh_render_flat(bh_ctx* ctx, const bh_flat_scene* sc, const bh_outputs* out) 
     if (out->phi_end) { if ((rc = ensure(ctx, ctx->phi, npix * 8))) return rc; o.phi = (double*)ctx->phi.p; }
     if (out->hit_point) { if ((rc = ensure(ctx, ctx->hitpt, npix * 24))) return rc; o.hitpt = (double*)ctx->hitpt.p; }
     if (out->steps) { if ((rc = ensure(ctx, ctx->steps, npix * 4))) return rc; o.steps = (int32_t*)ctx->steps.p; }
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     HIP_TRY(ctx, bh::launch_flat(d, o, st));
     if (out->rgb) HIP_TRY(ctx, hipMemcpyAsync(out->rgb, o.rgb, npix * 3, hipMemcpyDeviceToHost, st));
     if (out->hit) HIP_TRY(ctx, hipMemcpyAsync(out->hit, o.hit, npix, hipMemcpyDeviceToHost, st));
@@ -1679,7 +1717,7 @@ int bh_time_flat(bh_ctx* ctx, const bh_flat_scene* sc, int iters, double* avg_ms
     if ((rc = ensure(ctx, ctx->rgb, npix * 3))) return rc;
     if ((rc = ensure(ctx, ctx->hit, npix))) return rc;
     DevOut o{(uint8_t*)ctx->rgb.p, (uint8_t*)ctx->hit.p, nullptr, nullptr, nullptr};
-    hipStream_t st = ctx->stream;
+    hipStream_t st = work_stream(ctx);
     HIP_TRY(ctx, bh::launch_flat(d, o, st));  // warm-up
     HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
     for (int it = 0; it < iters; ++it) HIP_TRY(ctx, bh::launch_flat(d, o, st));

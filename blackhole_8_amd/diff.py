@@ -52,8 +52,8 @@ class DiffRenderer:
     included, so they follow the torch ops before and precede those after
     without events (with a stream of this object's own and two event waits a
     call, a 512x512 forward took 51 us and an image with its gradient 227;
-    here 19 and 142, of which the kernels are 18 and 51).  The context's other
-    calls run on a stream of this object."""
+    here 19 and 142, of which the kernels are 18 and 51).  The context keeps
+    its own stream for its other calls, which these calls follow and precede."""
 
     def __init__(self, renderer: Renderer, cfg: DiffConfig | None = None):
         if not torch.cuda.is_available():
@@ -61,19 +61,13 @@ class DiffRenderer:
         self.r = renderer
         self.cfg = cfg or DiffConfig()
         self.dev = torch.device("cuda", torch.cuda.current_device())
-        self.stream = torch.cuda.Stream(self.dev)
-        self._handle = C.c_void_p(self.stream.cuda_stream)
         self._ovf = torch.zeros(1, dtype=torch.int32, device=self.dev)
-
-    def _bind(self):
-        self.r._check(self.r.lib.bh_ctx_set_stream(self.r.ctx, self._handle))
 
     def forward(self, theta, with_hit: bool = False):
         c = self.cfg
         p = c.params(theta)
         rgb = torch.empty((c.height, c.width, 3), dtype=torch.float32, device=self.dev)
         hit = torch.empty((c.height, c.width), dtype=torch.uint8, device=self.dev) if with_hit else None
-        self._bind()
         self.r._check(self.r.lib.bh_diff_render_stream(
             self.r.ctx, torch.cuda.current_stream(self.dev).cuda_stream, C.byref(p), c.precision,
             rgb.data_ptr(), hit.data_ptr() if hit is not None else None))
@@ -92,7 +86,6 @@ class DiffRenderer:
         grad = torch.empty(4, dtype=torch.float64, device=self.dev)
         n = self.r.lib.bh_diff_work_bytes(c.width, c.height)
         work = torch.empty(n, dtype=torch.uint8, device=self.dev)
-        self._bind()
         cur = torch.cuda.current_stream(self.dev)
         g.record_stream(cur)
         self._ovf.record_stream(cur)
@@ -111,7 +104,6 @@ class DiffRenderer:
         f, a = C.c_double(), C.c_double()
         p = self.cfg.params(theta)
         torch.cuda.synchronize(self.dev)
-        self._bind()
         self.r._check(self.r.lib.bh_diff_time(self.r.ctx, C.byref(p), self.cfg.precision, iters,
                                               C.byref(f), C.byref(a)))
         return f.value, a.value

@@ -214,7 +214,11 @@ const char* bh_last_error(const bh_ctx* ctx);
 /* Library version and the device name / CU count the context runs on. */
 int bh_version(void);
 int bh_device_info(bh_ctx* ctx, char* name, int name_len, int* n_cu, int* clock_khz);
-/* Run the context's work on a caller stream (hipStream_t), NULL = own stream. */
+/* Run the context's work on a caller stream (hipStream_t), NULL = own stream.
+ * A context's calls share its scratch memory and follow each other in the order
+ * they are made, also from one stream to the next (but for captured calls and
+ * what they replay, which the caller orders).  A stream stays valid while it is
+ * the context's and until the work that calls put on it has ended. */
 int bh_ctx_set_stream(bh_ctx* ctx, void* stream);
 int bh_synchronize(bh_ctx* ctx);
 
@@ -397,10 +401,10 @@ int bh_diff_adjoint_device(bh_ctx* ctx, const bh_diff_params* p, int precision,
                            double* grad_out, uint32_t* overflow_out);
 /* The two calls on a stream of the caller's (hipStream_t; NULL is the null
  * stream) in place of the context's: a caller whose buffers belong to that
- * stream needs no events around the call.  They start after the work that the
- * context's stream holds (not under capture), and the context keeps nothing of
- * them: work is the caller's, bh_diff_work_bytes long and 8-aligned, and in use
- * until the call's work has ended. */
+ * stream needs no events around the call.  They keep the order of the
+ * context's calls (bh_ctx_set_stream), and the context keeps nothing of them:
+ * work is the caller's, bh_diff_work_bytes long and 8-aligned, and in use until
+ * the call's work has ended. */
 int bh_diff_render_stream(bh_ctx* ctx, void* stream, const bh_diff_params* p, int precision,
                           float* rgb_out, uint8_t* hit_out);
 size_t bh_diff_work_bytes(int width, int height);
