@@ -153,7 +153,9 @@ bool capturing(hipStream_t st) {
   return true;
 }
 
-// st waits for what `before` holds.
+// st waits for what `before` holds.  Neither may be capturing: a capturing
+// stream's state is not to be asked for, and an event of it would draw st into
+// the capture.
 void follow(bh_ctx* ctx, hipStream_t st, hipStream_t before) {
   if (hipStreamQuery(before) == hipSuccess) return;
   (void)hipGetLastError();
@@ -768,7 +770,7 @@ void enter_stream(bh_ctx* ctx, hipStream_t st) {
   ctx->other_streams = true;
   if (capturing(st)) return;
   follow_tail(ctx, st);
-  if (ctx->work) follow(ctx, st, ctx->stream);
+  if (ctx->work && !capturing(ctx->stream)) follow(ctx, st, ctx->stream);
   ctx->work = false;
   ctx->tail_stream = st;
   ctx->tail = true;
@@ -926,7 +928,7 @@ int bh_ctx_set_stream(bh_ctx* ctx, void* stream) {
     if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
     (void)hipSetDevice(ctx->device);
     const hipStream_t st = stream ? (hipStream_t)stream : ctx->own;
-    if (ctx->stream == ctx->own) {
+    if (ctx->stream == ctx->own && !capturing(st)) {
       (void)hipStreamSynchronize(ctx->own);
       ctx->work = false;
     } else if (ctx->stream != st && ctx->work) {

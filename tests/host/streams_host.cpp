@@ -41,6 +41,7 @@ struct Stream {
 };
 struct Event {
   Clock clock;
+  bool captured = false;
 };
 struct Launch {
   std::string what;
@@ -53,6 +54,16 @@ std::map<hipStream_t, Stream> streams;
 Clock host;  // what the host has waited for
 std::vector<Launch> launches;
 int next_id = 1;
+int refused = 0;  // calls that a capture does not allow
+
+// What a capture refuses: the state of a capturing stream, and waits of the
+// host and frees while any stream captures.
+bool refuse(hipStream_t st, bool any) {
+  bool no = streams[st].capturing;
+  for (const auto& [h, s] : streams) no = no || (any && s.capturing);
+  refused += no;
+  return no;
+}
 
 Stream& at(hipStream_t s) { return streams[s]; }
 
@@ -131,13 +142,21 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t, hipMemcpyKind, hipStre
 hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = new_stream(); return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { merge(host, at(s).clock); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) {
+  return refuse(s, true) ? hipErrorStreamCaptureUnsupported : hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (refuse(s, true)) return hipErrorStreamCaptureUnsupported;
+  merge(host, at(s).clock);
+  return hipSuccess;
+}
 hipError_t hipDeviceSynchronize() {
+  if (refuse(nullptr, true)) return hipErrorStreamCaptureUnsupported;
   for (auto& [h, s] : streams) merge(host, s.clock);
   return hipSuccess;
 }
 hipError_t hipStreamQuery(hipStream_t s) {
+  if (refuse(s, false)) return hipErrorStreamCaptureUnsupported;
   return covers(host, at(s).clock) ? hipSuccess : hipErrorNotReady;
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* c) {
@@ -145,6 +164,8 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* c) {
   return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  // (a wait for captured work draws the stream into the capture)
+  at(s).capturing = at(s).capturing || ((Event*)e)->captured;
   merge(at(s).clock, ((Event*)e)->clock);
   return hipSuccess;
 }
@@ -153,6 +174,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCre
 hipError_t hipEventDestroy(hipEvent_t e) { delete (Event*)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   ((Event*)e)->clock = at(s).clock;
+  ((Event*)e)->captured = at(s).capturing;
   return hipSuccess;
 }
 hipError_t hipEventQuery(hipEvent_t e) {
@@ -281,6 +303,7 @@ struct Setup {
     host.clear();
     launches.clear();
     next_id = 1;
+    refused = 0;
     at(nullptr).id = 0;
     if (bh_ctx_create(0, &ctx)) abort();
     memset(&sc, 0, sizeof sc);
@@ -361,6 +384,29 @@ bool calls_keep_their_order() {
   return ok && conflicts() == 0;
 }
 
+// The first image and gradient of a context under capture, the context's
+// stream set to the capturing one and a frame on it; then a frame after it.
+bool first_calls_in_a_capture() {
+  Setup s;
+  const hipStream_t c = new_stream();
+  bool ok = s.frame(s.rgb1);
+  at(c).capturing = true;
+  ok = ok && s.image_on(c) && s.adjoint_on(c) && s.set(c) && s.frame(s.rgb2) && refused == 0;
+  at(c).capturing = false;
+  return ok && s.frame(s.rgb1) && conflicts() == 0 && refused == 0;
+}
+
+// An image on a stream that does not capture while the context's stream does.
+bool image_beside_a_capture() {
+  Setup s;
+  const hipStream_t a = new_stream(), b = new_stream();
+  bool ok = s.set(a) && s.frame(s.rgb1);
+  at(a).capturing = true;
+  ok = ok && s.image_on(b) && refused == 0 && !at(b).capturing;
+  at(a).capturing = false;
+  return ok && s.frame(s.rgb2) && follows("scene", "diff") && conflicts() == 0;
+}
+
 }  // namespace
 
 int main() {
@@ -372,6 +418,8 @@ int main() {
       {"frames_on_two_streams", frames_on_two_streams},
       {"batches_on_two_streams", batches_on_two_streams},
       {"calls_keep_their_order", calls_keep_their_order},
+      {"first_calls_in_a_capture", first_calls_in_a_capture},
+      {"image_beside_a_capture", image_beside_a_capture},
   };
   int bad = 0;
   for (const auto& t : all) {

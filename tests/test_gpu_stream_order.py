@@ -60,3 +60,39 @@ def test_frames_between_images(r, moves):
         assert np.array_equal(rgb.cpu().numpy(), solo["rgb"]), k
         assert np.array_equal(hit.cpu().numpy(), solo["hit"]), k
         assert torch.equal(images[k].cpu(), want), k
+
+
+def test_first_calls_of_a_context_in_a_capture():
+    """A new context whose first image and gradient, and whose move to the
+    capturing stream, come inside a capture; every replay equals the eager
+    calls."""
+    print("[case] first calls in a capture", flush=True)
+    p = scenes.disc_orbit(317, 179)
+    w, h = 130, 70
+    weights = (torch.rand((h, w, 3), generator=torch.Generator().manual_seed(2)) + 0.5).cuda()
+    frame = torch.zeros((179, 317, 3), dtype=torch.uint8, device="cuda")
+    o = abi.Outputs(frame.data_ptr())
+    graph = torch.cuda.CUDAGraph()
+    with Renderer(0) as own:
+        own.set_textures(p.textures)
+        dr = diff.DiffRenderer(own, diff.DiffConfig(width=w, height=h))
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            rgb = dr.forward(diff.FIT_START)
+            grad = dr.adjoint(diff.FIT_START, weights)
+            own._check(own.lib.bh_ctx_set_stream(
+                own.ctx, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+            own._check(own.lib.bh_render_device_noalloc(
+                own.ctx, C.byref(p.scene), C.byref(p.options), C.byref(o)))
+        own._check(own.lib.bh_ctx_set_stream(own.ctx, None))
+        want = dr.forward(diff.FIT_START).cpu()
+        want_grad = dr.adjoint(diff.FIT_START, weights).cpu()
+        solo = own.render(p.scene, p.options, ("rgb",))["rgb"]
+        for _ in range(3):
+            rgb.zero_(), grad.zero_(), frame.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(rgb.cpu(), want) and torch.equal(grad.cpu(), want_grad)
+            assert np.array_equal(frame.cpu().numpy(), solo)
+            assert torch.equal(dr.forward(diff.FIT_START).cpu(), want)
+        torch.cuda.synchronize()
