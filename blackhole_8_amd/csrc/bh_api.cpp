@@ -53,7 +53,7 @@ struct bh_ctx {
   // tail: the context's last work is on another stream, tail_stream
   hipStream_t tail_stream = nullptr;
   bool tail = false;
-  bool other_streams = false;  // a call has put work on a caller's stream
+  bool adrift = false;  // work that neither `stream` nor the tail covers (captures)
   char name[256] = {0};
   int n_cu = 0, clock_khz = 0;
 };
@@ -164,6 +164,14 @@ void follow(bh_ctx* ctx, hipStream_t st, hipStream_t before) {
     (void)hipGetLastError();
     (void)hipDeviceSynchronize();
   }
+}
+
+// Another stream than `stream` holds the context's last work.
+void set_tail(bh_ctx* ctx, hipStream_t st) {
+  ctx->adrift = ctx->adrift || (ctx->tail && ctx->tail_stream != st);  // one not followed
+  ctx->tail_stream = st;
+  ctx->tail = true;
+  ctx->work = false;
 }
 
 // st waits for the tail, if there is one.
@@ -767,21 +775,40 @@ void enter_stream(bh_ctx* ctx, hipStream_t st) {
     (void)work_stream(ctx);
     return;
   }
-  ctx->other_streams = true;
-  if (capturing(st)) return;
+  if (capturing(st)) {  // (its replays may still run at the next wait for the context)
+    ctx->adrift = true;
+    return;
+  }
   follow_tail(ctx, st);
-  if (ctx->work && !capturing(ctx->stream)) follow(ctx, st, ctx->stream);
-  ctx->work = false;
-  ctx->tail_stream = st;
-  ctx->tail = true;
+  if (ctx->work) {
+    if (capturing(ctx->stream))
+      ctx->adrift = true;
+    else
+      follow(ctx, st, ctx->stream);
+  }
+  set_tail(ctx, st);
 }
 
-// Waits for all work the context's calls have put on the device.
+// Waits for all work the context's calls have put on the device: for the streams
+// that hold it, and for the whole device only where captures were about or a
+// caller has destroyed its stream.
 hipError_t context_idle(bh_ctx* ctx) {
-  if (!ctx->other_streams) return hipStreamSynchronize(ctx->stream);
-  const hipError_t e = hipDeviceSynchronize();
-  if (e == hipSuccess) ctx->other_streams = false;
-  return e;
+  hipError_t e = hipStreamSynchronize(ctx->stream);
+  if (e != hipSuccess) return e;
+  if (ctx->tail && hipStreamSynchronize(ctx->tail_stream) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->adrift = true;
+  }
+  if (ctx->adrift) {
+    int current = ctx->device;
+    (void)hipGetDevice(&current);
+    (void)hipSetDevice(ctx->device);
+    e = hipDeviceSynchronize();
+    (void)hipSetDevice(current);
+    if (e != hipSuccess) return e;
+  }
+  ctx->work = ctx->tail = ctx->adrift = false;
+  return hipSuccess;
 }
 
 int diff_render_on(bh_ctx* ctx, hipStream_t st, const bh_diff_params* p, int precision,
@@ -932,9 +959,7 @@ int bh_ctx_set_stream(bh_ctx* ctx, void* stream) {
       (void)hipStreamSynchronize(ctx->own);
       ctx->work = false;
     } else if (ctx->stream != st && ctx->work) {
-      ctx->tail_stream = ctx->stream;
-      ctx->tail = ctx->other_streams = true;
-      ctx->work = false;
+      set_tail(ctx, ctx->stream);
     }
     ctx->stream = st;
     return BH_OK;

@@ -37,7 +37,7 @@ bool covers(const Clock& a, const Clock& b) {
 struct Stream {
   int id = 0;
   Clock clock;
-  bool capturing = false;
+  bool capturing = false, dead = false;
 };
 struct Event {
   Clock clock;
@@ -122,6 +122,7 @@ bool follows(const char* b, const char* a) {
 extern "C" {
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
   memset(p, 0, sizeof *p);
   p->multiProcessorCount = 256;
@@ -143,9 +144,12 @@ hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; 
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = new_stream(); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) {
-  return refuse(s, true) ? hipErrorStreamCaptureUnsupported : hipSuccess;
+  if (refuse(s, true)) return hipErrorStreamCaptureUnsupported;
+  at(s).dead = true;
+  return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (at(s).dead) return hipErrorContextIsDestroyed;
   if (refuse(s, true)) return hipErrorStreamCaptureUnsupported;
   merge(host, at(s).clock);
   return hipSuccess;
@@ -156,14 +160,17 @@ hipError_t hipDeviceSynchronize() {
   return hipSuccess;
 }
 hipError_t hipStreamQuery(hipStream_t s) {
+  if (at(s).dead) return hipErrorContextIsDestroyed;
   if (refuse(s, false)) return hipErrorStreamCaptureUnsupported;
   return covers(host, at(s).clock) ? hipSuccess : hipErrorNotReady;
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* c) {
+  if (at(s).dead) return hipErrorContextIsDestroyed;
   *c = at(s).capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  if (at(s).dead) return hipErrorContextIsDestroyed;
   // (a wait for captured work draws the stream into the capture)
   at(s).capturing = at(s).capturing || ((Event*)e)->captured;
   merge(at(s).clock, ((Event*)e)->clock);
@@ -173,6 +180,7 @@ hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t) new Event; return h
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete (Event*)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (at(s).dead) return hipErrorContextIsDestroyed;
   ((Event*)e)->clock = at(s).clock;
   ((Event*)e)->captured = at(s).capturing;
   return hipSuccess;
@@ -407,6 +415,26 @@ bool image_beside_a_capture() {
   return ok && s.frame(s.rgb2) && follows("scene", "diff") && conflicts() == 0;
 }
 
+// A wait for the context's work (a texture about to be replaced) covers all of
+// it and no other stream's, also once a caller has destroyed its stream.
+bool waits_for_its_own_work() {
+  Setup s;
+  const hipStream_t a = new_stream(), b = new_stream(), c = new_stream(), x = new_stream();
+  uint8_t texel[3] = {1, 2, 3};
+  const bh_image img{texel, 1, 1, 3};
+  const auto done = [](hipStream_t st) { return covers(host, at(st).clock); };
+  launch("other", x, {}, {});
+  bool ok = s.set(a) && s.frame(s.rgb1) && s.set(b) && s.image_on(c);
+  ok = ok && bh_texture_set(s.ctx, 1, &img) == BH_OK && done(a) && done(c) && !done(x);
+  ok = ok && s.frame(s.rgb1) && s.set(a) && bh_synchronize(s.ctx) == BH_OK && done(b) && !done(x);
+  ok = ok && s.image_on(c) && s.adjoint_on(b) && bh_texture_clear(s.ctx, 1) == BH_OK && done(b) &&
+       done(c) && !done(x);
+  ok = ok && s.image_on(c) && hipStreamSynchronize(c) == hipSuccess &&
+       hipStreamDestroy(c) == hipSuccess;
+  return ok && bh_texture_set(s.ctx, 1, &img) == BH_OK && s.image_on(b) && s.frame(s.rgb2) &&
+         bh_synchronize(s.ctx) == BH_OK && done(a) && done(b);
+}
+
 }  // namespace
 
 int main() {
@@ -420,6 +448,7 @@ int main() {
       {"calls_keep_their_order", calls_keep_their_order},
       {"first_calls_in_a_capture", first_calls_in_a_capture},
       {"image_beside_a_capture", image_beside_a_capture},
+      {"waits_for_its_own_work", waits_for_its_own_work},
   };
   int bad = 0;
   for (const auto& t : all) {
