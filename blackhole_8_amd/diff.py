@@ -61,7 +61,9 @@ class DiffRenderer:
         self.r = renderer
         self.cfg = cfg or DiffConfig()
         self.dev = torch.device("cuda", torch.cuda.current_device())
+        # the last adjoint's count of overflowed rays and its stream
         self._ovf = torch.zeros(1, dtype=torch.int32, device=self.dev)
+        self._ovf_stream = torch.cuda.current_stream(self.dev)
 
     def forward(self, theta, with_hit: bool = False):
         c = self.cfg
@@ -86,17 +88,22 @@ class DiffRenderer:
         grad = torch.empty(4, dtype=torch.float64, device=self.dev)
         n = self.r.lib.bh_diff_work_bytes(c.width, c.height)
         work = torch.empty(n, dtype=torch.uint8, device=self.dev)
+        # a word of its own a call: calls on several streams run in any order
+        ovf = torch.empty(1, dtype=torch.int32, device=self.dev)
         cur = torch.cuda.current_stream(self.dev)
         g.record_stream(cur)
-        self._ovf.record_stream(cur)
         self.r._check(self.r.lib.bh_diff_adjoint_stream(
             self.r.ctx, cur.cuda_stream, C.byref(p), c.precision, g.data_ptr(),
             rgb.data_ptr() if rgb is not None else None, None, grad.data_ptr(),
-            self._ovf.data_ptr(), work.data_ptr(), n))
+            ovf.data_ptr(), work.data_ptr(), n))
+        self._ovf, self._ovf_stream = ovf, cur
         return (grad, rgb) if want_rgb else grad
 
     def overflow(self) -> int:
         """Rays of the last adjoint whose disc crossings exceeded the record."""
+        cur = torch.cuda.current_stream(self.dev)
+        if cur != self._ovf_stream:
+            cur.wait_stream(self._ovf_stream)
         return int(self._ovf.item())
 
     def time(self, theta, iters: int = 20):
