@@ -834,9 +834,9 @@ int diff_adjoint_scene(bh_ctx* ctx, const bh_diff_params* p, int precision, cons
 
 // Fused path launches: the queue counts cleared, every frame's march in one
 // launch (up to 1024 frames each), then every frame's FP64 band pass in one
-// launch.  The clearing launch stays out of the march's graph, whose timing
-// events bracket the march alone (launch to end of 24 480x270 frames: 122 us
-// as a second node, 118 beside it).
+// launch.  The clearing launch stays out of the march's graph (launch to end of
+// 24 480x270 frames: 122 us as a second node, 118 beside it) and inside its
+// timing events.
 constexpr int kFramesPerLaunch = 1024;
 
 hipError_t path_clear(const bh_path* p, hipStream_t st) {
@@ -1285,8 +1285,8 @@ int bh_path_launch(bh_path* p, float* ms) {
     hipStream_t st = work_stream(ctx);
     if (p->exec_band) {
       // the march graph, then the FP64 pass's, with timing events around each
-      HIP_TRY(ctx, path_clear(p, st));
       HIP_TRY(ctx, hipEventRecord(p->k0, st));
+      HIP_TRY(ctx, path_clear(p, st));
       HIP_TRY(ctx, hipGraphLaunch(p->exec, st));
       HIP_TRY(ctx, hipEventRecord(p->k1, st));
       HIP_TRY(ctx, hipGraphLaunch(p->exec_band, st));
@@ -1388,8 +1388,8 @@ int bh_path_time(bh_path* p, int iters, double* march_ms, double* band_ms) {
     hipStream_t st = work_stream(ctx);
     double tm = 0, tb = 0;
     for (int it = 0; it < iters; ++it) {
-      HIP_TRY(ctx, path_clear(p, st));
       HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
+      HIP_TRY(ctx, path_clear(p, st));
       HIP_TRY(ctx, path_march(p, st));
       HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
       HIP_TRY(ctx, path_band(p, st));

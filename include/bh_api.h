@@ -279,13 +279,14 @@ int bh_path_create(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
  * one graph of per-frame launches. */
 int bh_path_launch(bh_path* path, float* ms);
 /* Average ms of those two launches over iters eager runs (HIP events on the
- * context stream); BH_ERR_UNSUPPORTED for paths with FP64 frames. */
+ * context stream; the march's with the small launch that clears its queue
+ * counts); BH_ERR_UNSUPPORTED for paths with FP64 frames. */
 int bh_path_time(bh_path* path, int iters, double* march_ms, double* band_ms);
-/* The durations (ms) of the fused march launch and of the FP64 pass in the
- * path's last bh_path_launch, from HIP events on the context stream around
- * each (a path whose frames all take the FP32 march is two graphs, the march
- * over all frames and the FP64 pass over all frames, launched back to back).
- * Other paths: BH_ERR_UNSUPPORTED. */
+/* The durations (ms) of the fused march launch (and its clearing launch) and of
+ * the FP64 pass in the path's last bh_path_launch, from HIP events on the
+ * context stream around each (a path whose frames all take the FP32 march is two
+ * graphs, the march over all frames and the FP64 pass over all frames, launched
+ * back to back).  Other paths: BH_ERR_UNSUPPORTED. */
 int bh_path_last_ms(bh_path* path, double* march_ms, double* band_ms);
 /* Copy frame i back to host buffers (rgb H*W*3, hit H*W; either may be NULL). */
 int bh_path_read(bh_path* path, int frame, uint8_t* rgb, uint8_t* hit);

@@ -189,7 +189,13 @@ hipError_t hipEventQuery(hipEvent_t e) {
   return covers(host, ((Event*)e)->clock) ? hipSuccess : hipErrorNotReady;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) { merge(host, ((Event*)e)->clock); return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }
+// (every launch takes 1 ms)
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
+  *ms = 0.f;
+  for (const auto& [k, v] : ((Event*)b)->clock) *ms += (float)v;
+  for (const auto& [k, v] : ((Event*)a)->clock) *ms -= (float)v;
+  return hipSuccess;
+}
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { at(s).capturing = true; return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
   at(s).capturing = false;
@@ -435,6 +441,24 @@ bool waits_for_its_own_work() {
          bh_synchronize(s.ctx) == BH_OK && done(a) && done(b);
 }
 
+// The reported times of a path's replay hold all its launches.
+bool path_times_hold_every_launch() {
+  Setup s;
+  const bh_camera cams[2] = {s.sc.camera, s.sc.camera};
+  bh_path* p = nullptr;
+  if (bh_path_create(s.ctx, &s.sc, &s.opt, cams, 2, &p) != BH_OK) return false;
+  float ms = 0.f;
+  double march = 0.0, band = 0.0, march2 = 0.0, band2 = 0.0;
+  const size_t n0 = launches.size();
+  bool ok = bh_path_launch(p, &ms) == BH_OK && bh_path_last_ms(p, &march, &band) == BH_OK;
+  const size_t n1 = launches.size();
+  ok = ok && bh_path_time(p, 1, &march2, &band2) == BH_OK;
+  const size_t n2 = launches.size();
+  bh_path_destroy(p);
+  return ok && n1 > n0 && ms == (float)(n1 - n0) && march + band == (double)(n1 - n0) &&
+         march2 + band2 == (double)(n2 - n1);
+}
+
 }  // namespace
 
 int main() {
@@ -449,6 +473,7 @@ int main() {
       {"first_calls_in_a_capture", first_calls_in_a_capture},
       {"image_beside_a_capture", image_beside_a_capture},
       {"waits_for_its_own_work", waits_for_its_own_work},
+      {"path_times_hold_every_launch", path_times_hold_every_launch},
   };
   int bad = 0;
   for (const auto& t : all) {
