@@ -644,8 +644,8 @@ int run_batch(bh_ctx* ctx, const BatchPlan& p, const bh_batch_tuning& t, bool ti
       if (p.cls_tile[c + 1] - p.cls_tile[c] == p.cls_tile[4]) cls = c;
     HIP_TRY(ctx, bh::launch_batch_band(b, cls, st));
   }
-  // solo scenes: the per-frame kernels, with the context's band queue (the
-  // band kernel clears it after each scene)
+  // solo scenes: the per-frame kernels, with the context's queue (each scene's
+  // first launch clears its counts)
   if (!p.solo.empty()) {
     int maxw = 0, maxh = 0;
     for (int i : p.solo) {

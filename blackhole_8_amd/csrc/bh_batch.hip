@@ -374,7 +374,7 @@ __device__ inline bool march_tile_xy(const BatchDev& b, const DevScene& s,
       const double du = (r.l - s.u0) * s.inv_nstep;
       setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
       if constexpr (SPH) setup_spheres32(s, r, L);
-      march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
+      march<ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
       if constexpr (SPH) sredo = L.sredo;
     }
     redo = finish_ray<ESCAPE>(s, load_out(outp), idx, r, mo, phi0) || sredo;

@@ -427,7 +427,7 @@ template <typename T> struct Acc {
   T rgb[3];
   T tr;  // transmittance
   int cls, n;
-  bool done, overflow;
+  bool overflow;
   uint64_t mask;
 };
 
@@ -490,7 +490,6 @@ __device__ inline void diff_march(const DiffScene& s, const DRay<T>& d, const St
   a.tr = (T)1;
   a.cls = BH_HIT_NONE;
   a.n = 0;
-  a.done = false;
   a.overflow = false;
   a.mask = 0;
   if (d.degenerate) {  // pixel line through the centre: captured, black

@@ -45,11 +45,6 @@ __device__ __forceinline__ d3 pixel_point(const DevScene& s, int x, int y) {
   return (ld3(s.fv) - ld3(s.vy) * sx) - ld3(s.vz) * sy;
 }
 
-// StaticBlackhole::G (blackhole_solution.h:27-29)
-__device__ __forceinline__ double G64(double u, double b, double M) {
-  return (u * u * (2.0 * M * u - 1.0)) + (1.0 / (b * b));
-}
-
 // StaticBlackhole::SolveG (blackhole_solution.h:35-53); l0 = cbrt(eps_double)
 // is computed on the host.  BH_ROOT_EXACT bisects until the bracket stops
 // shrinking.  G is strictly decreasing on (0, 1/(3M)), so the decisions are

@@ -238,7 +238,8 @@ __device__ __forceinline__ uint32_t sphere_mask(const DevScene& s, Lane<double>&
   return mask;
 }
 
-// A sphere of radius R whose centre lies at distance z from the plane cuts it in a circle of radius sqrt(R^2 - z^2), and
+// A sphere of radius R whose centre lies at distance z from the plane cuts it in
+// a circle of radius sqrt(R^2 - z^2), and
 // |P - c|^2 = |P - c'|^2 + z^2 for a point P of the plane and the centre's
 // projection c', so the reference's segment/sphere test
 // (blackhole_solution.h:65-88, the same test as the horizon's) of an in-plane
@@ -470,10 +471,10 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
   return step_tests<T, S, SPH>(s, L, st, st.a - (double)st.d, first_aa, ka, kb, force, hit);
 }
 
-// The march of one FP32 ray.  first_aa is the angle of the camera
-// in the (e1, e2) frame: 0 when Y0 > 0, pi when Y0 < 0 (the reference's
-// phi0 = atan(b/Y0) then points away from the camera, and only the first
-// chord starts at the camera itself).
+// The march of one FP32 ray (FP64 ones take march64e).  first_aa is the angle
+// of the camera in the (e1, e2) frame: 0 when Y0 > 0, pi when Y0 < 0 (the
+// reference's phi0 = atan(b/Y0) then points away from the camera, and only the
+// first chord starts at the camera itself).
 //
 // Every lane of a wave is at the same step, so the loops run wave-uniform
 // trip counts and keep no per-lane flag: a ray that has ended is disarmed by
@@ -497,18 +498,18 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
 //    r cos(d/2) >= r (1 - d^2/8).
 // A wave of a disc seen from 20 r_s at 10 degrees took 27.3 steps on average
 // and takes 21.7.
-template <typename T, bool ESCAPE, bool SPH = false, int NS = 0>
-__device__ inline void march(const DevScene& s, Lane<T>& L, bool captured, double first_aa,
-                             double du64, bool brief, MarchOut<T>& o) {
+template <bool ESCAPE, bool SPH = false, int NS = 0>
+__device__ inline void march(const DevScene& s, Lane<float>& L, bool captured, double first_aa,
+                             double du64, bool brief, MarchOut<float>& o) {
+  using T = float;
   // NS > 0: the scene's nstep, known at compile time: the blocks unroll, and
   // their step values and chord ends become literal operands (no per-step
   // integer-to-float conversion, no loop bookkeeping)
   const int nstep = NS > 0 ? NS : s.nstep;
-  // block length: six steps in the compiled instance of an FP32 lane
-  // without sphere slots (fewer checks and single tail steps: 20 steps leave
-  // none inbound and one outbound; nine-step blocks measured no faster and
-  // spill), four otherwise (six would cost the sphere lanes occupancy)
-  static_assert(sizeof(T) == 4, "FP64 lanes take march64e");
+  // block length: six steps in the compiled instance without sphere slots
+  // (fewer checks and single tail steps: 20 steps leave none inbound and one
+  // outbound; nine-step blocks measured no faster and spill), four otherwise
+  // (six would cost the sphere lanes occupancy)
   constexpr int kB = (NS > 0 && !SPH) ? 6 : 4;
   MarchState<T> st{(T)0, 0.0, (T)0};
   o.hit.cls = BH_HIT_NONE;

@@ -7,8 +7,11 @@
 //                  an object can be reached; rays in the photon-sphere band,
 //                  and rays whose texel lies within the edge guard of a texel
 //                  edge, are queued for band_kernel.
-//  band_kernel     the FP64 reference march (march64_kernel's per-pixel code)
-//                  of the queued rays.
+//  band_kernel     the queued rays in FP64: the event march's outcome refined, or
+//                  its event march in FP64, settled where the last bits count by
+//                  the reference march (march64_kernel's per-pixel code).
+//  scene_kernel    a frame's first launch: its scene record in place, its queue
+//                  counts cleared.
 //  march_frames_kernel / band_frames_kernel
 //                  the same two passes over every frame of a camera path in
 //                  one launch each.
@@ -71,7 +74,7 @@ __device__ __forceinline__ void march_pixel(const DevScene& s, const DevOut& out
     const double du = (r.l - s.u0) * s.inv_nstep;
     setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
     if constexpr (SPH) setup_spheres32(s, r, L);
-    march<float, ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
+    march<ESCAPE, SPH, NS>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
     if constexpr (SPH) sredo = L.sredo;
   }
   // the texel lies within the FP32 error of a texel edge (or a sphere was
@@ -350,7 +353,6 @@ hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t stream) {
 }
 
 hipError_t launch_scene(const DevScene& s, DevScene* dst, uint32_t* count, hipStream_t stream) {
-  static_assert(sizeof(DevScene) % 4 == 0, "scene record is copied as 32-bit words");
   static_assert(sizeof(DevScene) + 2 * sizeof(void*) <= 4096,
                 "the scene record is passed as a kernel argument");
   hipLaunchKernelGGL(scene_kernel, dim3(1), dim3(kSceneThreads), 0, stream, s, dst, count);

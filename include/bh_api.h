@@ -351,7 +351,7 @@ typedef struct bh_batch_tuning {
 } bh_batch_tuning;
 
 typedef struct bh_batch_stats {
-  double total_ms;    /* upload of the batch tables to completion (HIP events) */
+  double total_ms;    /* the march's first launch to completion (HIP events)  */
   double march_ms;    /* persistent FP32 march                                 */
   double band_ms;     /* FP64 photon-sphere band pass                          */
   int64_t rays;       /* pixels rendered                                       */
@@ -363,7 +363,8 @@ typedef struct bh_batch_stats {
 /* Render n scenes; scene i with options[i] into outs[i] (device pointers,
  * planes as for bh_render_device).  Every scene's output equals its own
  * bh_render_device output.  Scenes the FP32 march does not take (FP64,
- * spheres, bilinear) are rendered one by one after the batch.  scene_ms
+ * bilinear; in the lanes mode also those with spheres) are rendered one by one
+ * after the batch.  scene_ms
  * (host, n doubles, optional) receives each scene's completion time from the
  * start of the march; with scene_ms or stats the call waits for completion,
  * otherwise it is asynchronous on the context stream. */
