@@ -10,12 +10,15 @@ FP32 error of a texel edge.  Inputs are resident in HBM before the timed
 region; outputs stay in HBM.
 
 Prints one JSON line.  `roofline` covers the dominant kernel (the FP32
-march, every frame of the path in one launch): algorithmic FLOPs of the
-path (blackhole_8_amd/flops.py, from each frame's own per-pixel step counts)
-over that launch's HIP-event duration on the context stream, against the
-FP32 vector peak; beside it the FMA throughput a plain (not packed) FP32
-instruction stream reaches on this device, measured here (bh_fma_issue_rate),
-and the march's VALU busy fraction from rocprof counters (profiles/).
+march, every frame of the path in one launch): algorithmic FLOPs of the steps
+that it takes of each ray (blackhole_8_amd/flops.py, bh_steps_taken) over that
+launch's HIP-event duration on the context stream, against the FP32 vector
+peak.  Beside it, from rocprof counters (profiles/), the floating-point
+operations that the launch issues, against the FMA throughput a plain (not
+packed) FP32 instruction stream reaches on this device, measured here
+(bh_fma_issue_rate), and its VALU busy fraction.  `reference_equivalent_tflops`
+charges every ray the steps of the reference's rule, also where its march ends
+early: a speed, not a rate of the hardware.
 `accuracy` compares frames 0, 59 and 119 of the timed graph's own output
 with the FP64 oracle.  `spheres` gives the same roofline for the 720p
 16-sphere scene's march kernel (march_kernel<true,true,20>) and its whole-frame
@@ -78,10 +81,12 @@ def batch_timing(reps: int = 3) -> dict:
         ms0, st0 = best_of(None)
         best, rec = tune.autotune(r, items, reps=2)
         ms1, st1 = best_of(best)
-        # algorithmic work of the batch, from every scene's own steps and hits
+        # the batch's work: of the steps taken, and by the reference's rule
         outs = r.render_batch(items, want=("hit", "steps"))
-        flop = sum(flops.frame_flops(o["steps"], o["hit"], bool(s.has_disc))
-                   for o, (s, _) in zip(outs, items))
+        ref_flop = sum(flops.frame_flops(o["steps"], o["hit"], bool(s.has_disc))
+                       for o, (s, _) in zip(outs, items))
+        flop = sum(flops.taken_flops(r.steps_taken(s, opt), o["hit"], bool(s.has_disc))
+                   for o, (s, opt) in zip(outs, items))
     finally:
         r.close()
 
@@ -91,6 +96,7 @@ def batch_timing(reps: int = 3) -> dict:
                 "band_ms": round(st.band_ms, 4), "band_rays": int(st.band_rays),
                 "mrays_per_s": round(rays / st.total_ms / 1e3, 1),
                 "march_tflops": round(tf, 2), "frac_fp32_peak": round(tf / FP32_PEAK_TFLOPS, 4),
+                "reference_equivalent_tflops": round(ref_flop / (st.march_ms * 1e-3) / 1e12, 2),
                 "scene_ms_median": round(float(np.median(ms)), 4),
                 "scene_ms_p90": round(float(np.quantile(ms, 0.9)), 4),
                 "scene_ms_max": round(float(ms.max()), 4)}
@@ -99,6 +105,7 @@ def batch_timing(reps: int = 3) -> dict:
                         "U[6,50] r_s, inclination U[0,90] deg, disc with p 0.5, FP32, one "
                         "batch call (grid, persistent-tile or lane-refill mode, autotuned)",
             "scenes": len(items), "rays": int(rays), "algorithmic_gflop": round(flop / 1e9, 2),
+            "reference_equivalent_gflop": round(ref_flop / 1e9, 2),
             "default": line(ms0, st0),
             "tuned": dict(line(ms1, st1), tuning={f: getattr(best, f)
                                                    for f, _ in best._fields_})}
@@ -341,14 +348,18 @@ def main() -> int:
     # All frames of the path march in one launch (march_frames_kernel); its
     # duration is the mean over the timed replays of the HIP events the graph
     # records on the context stream around that kernel (bh_path_last_ms), the
-    # work comes from each frame's own per-pixel step counts and hit classes.
+    # work comes from the steps it takes of each frame's rays and their classes.
     march_ms, band_ms = march_sum / args.steps, band_sum / args.steps
-    work, band = 0.0, 0
+    work = ref_work = 0.0
+    taken = 0
     alg_bytes = 0  # framebuffer (3 B rgb + 1 B class) and one 4-byte texel per disc hit
     for k in range(F):
         sc = p.with_camera(p.cameras[k]).scene
         out = r.render(sc, p.options, ("hit", "steps"))
-        work += flops.frame_flops(out["steps"], out["hit"], True)
+        steps = r.steps_taken(sc, p.options)
+        work += flops.taken_flops(steps, out["hit"], True)
+        ref_work += flops.frame_flops(out["steps"], out["hit"], True)
+        taken += int(steps.sum())
         alg_bytes += W * H * 4 + 4 * int((out["hit"] == abi.HIT_DISC).sum())
     single = [r.time_render(p.with_camera(p.cameras[k]).scene, p.options, iters=4)
               for k in (0, F // 2)]
@@ -363,12 +374,17 @@ def main() -> int:
             traffic = json.loads(TRAFFIC_FILE.read_text()).get("bytes_per_launch")
         except (OSError, ValueError):
             traffic = None
-    valu = None
+    valu = issued = None
     if VALU_FILE.exists():
         try:
-            valu = json.loads(VALU_FILE.read_text()).get("valu_busy")
+            counters = json.loads(VALU_FILE.read_text())
+            valu = counters.get("valu_busy")
+            issued = counters.get("issued_flop_per_launch")
         except (OSError, ValueError):
-            valu = None
+            valu = issued = None
+    if F != 120:
+        issued = None  # counted for the launch of 120 frames
+    issued_tflops = issued / (march_ms * 1e-3) / 1e12 if issued else None
     roofline = {
         "bound": "valu",
         "kernel": "march_frames_kernel<false,false,20> (FP32 event march compiled for the reference's 20 steps, all frames in one launch)",
@@ -378,7 +394,8 @@ def main() -> int:
         "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
         "fp32_fma_issue_tflops": round(fma32.value, 2),
         "fp64_fma_issue_tflops": round(fma64.value, 2),
-        "frac_of_fma_issue": round(achieved / fma32.value, 4),
+        "issued_tflops": round(issued_tflops, 2) if issued else None,
+        "frac_of_fma_issue": round(issued_tflops / fma32.value, 4) if issued else None,
         "valu_busy": valu,
         "traffic": traffic,
         "traffic_per": "launch (all frames of the path)",
@@ -391,8 +408,10 @@ def main() -> int:
         "band_launch_ms": round(band_ms, 4),
         "single_frame_kernel_ms": round(sum(m for m, _, _ in single) / len(single), 5),
         "flop_per_frame": round(work / F),
-        "flop_basis": "steps of the reference rule, also of rays whose march ends early "
-                      "because nothing is left for them to meet",
+        "flop_basis": "the steps that the march takes of each ray (bh_steps_taken)",
+        "steps_taken_per_ray": round(taken / (W * H * F), 3),
+        "reference_equivalent_tflops": round(ref_work / (march_ms * 1e-3) / 1e12, 2),
+        "reference_flop_per_frame": round(ref_work / F),
         "band_rays_per_frame": round(sum(n for _, _, n in single) / len(single), 1),
     }
 

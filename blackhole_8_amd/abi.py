@@ -134,6 +134,8 @@ SIGNATURES = {
     "bh_chord_sincos": (C.c_int, [P, C.POINTER(C.c_float), C.POINTER(C.c_float), C.c_int64]),
     "bh_turning_points": (C.c_int, [P, C.POINTER(Scene), C.POINTER(Options),
                                     C.POINTER(C.c_double)]),
+    "bh_steps_taken": (C.c_int, [P, C.POINTER(Scene), C.POINTER(Options),
+                                 C.POINTER(C.c_int32)]),
     "bh_path_last_ms": (C.c_int, [P, C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "bh_path_create": (C.c_int, [P, C.POINTER(Scene), C.POINTER(Options), C.POINTER(Camera),
                                  C.c_int, C.POINTER(P)]),

@@ -1378,6 +1378,30 @@ int bh_turning_points(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
   });
 }
 
+int bh_steps_taken(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
+                   int32_t* steps_host) {
+  return guarded(ctx, [&]() -> int {
+    if (!ctx) return fail(nullptr, BH_ERR_BAD_HANDLE, "ctx is NULL");
+    if (!steps_host) return fail(ctx, BH_ERR_INVALID_ARG, "steps_host is NULL");
+    DevScene d;
+    int rc = build_scene(ctx, scene, opt, &d);
+    if (rc) return rc;
+    if (!fp32_eligible(d) || d.escape || d.n_spheres > 0)
+      return fail(ctx, BH_ERR_UNSUPPORTED, "only the FP32 march of holes and discs ends rays early");
+    (void)hipSetDevice(ctx->device);
+    const size_t bytes = (size_t)d.W * d.H * sizeof(int32_t);
+    if ((rc = ensure(ctx, ctx->scene, sizeof(DevScene)))) return rc;
+    if ((rc = ensure(ctx, ctx->steps, bytes))) return rc;
+    hipStream_t st = work_stream(ctx);
+    HIP_TRY(ctx, bh::launch_scene(d, (DevScene*)ctx->scene.p, nullptr, st));
+    HIP_TRY(ctx, bh::launch_steps_taken((const DevScene*)ctx->scene.p, (int32_t*)ctx->steps.p, d.W,
+                                        d.H, d.nstep, st));
+    HIP_TRY(ctx, hipMemcpyAsync(steps_host, ctx->steps.p, bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(ctx, hipStreamSynchronize(st));
+    return BH_OK;
+  });
+}
+
 int bh_path_time(bh_path* p, int iters, double* march_ms, double* band_ms) {
   return guarded(nullptr, [&]() -> int {
     if (!p) return fail(nullptr, BH_ERR_BAD_HANDLE, "path is NULL");

@@ -187,6 +187,8 @@ hipError_t launch_band_frames(const DevScene* scenes, const DevOut& out, int W, 
                               bool escape, bool spheres);
 hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t stream);
 hipError_t launch_turning(const DevScene* scene, double* l, int W, int H, hipStream_t stream);
+hipError_t launch_steps_taken(const DevScene* scene, int32_t* taken, int W, int H, int nstep,
+                              hipStream_t stream);
 
 // ---------------------------------------------------------------------------
 // Batch of independent FP32 scenes marched by one persistent launch.  Ray ids

@@ -498,7 +498,8 @@ __device__ __forceinline__ bool march_step(const S& s, Lane<T>& L, MarchState<T>
 //    r cos(d/2) >= r (1 - d^2/8).
 // A wave of a disc seen from 20 r_s at 10 degrees took 27.3 steps on average
 // and takes 21.7.
-template <bool ESCAPE, bool SPH = false, int NS = 0>
+// TAKEN (a measurement's instance): o.steps is the step it ended after.
+template <bool ESCAPE, bool SPH = false, int NS = 0, bool TAKEN = false>
 __device__ inline void march(const DevScene& s, Lane<float>& L, bool captured, double first_aa,
                              double du64, bool brief, MarchOut<float>& o) {
   using T = float;
@@ -652,7 +653,7 @@ __device__ inline void march(const DevScene& s, Lane<float>& L, bool captured, d
     }
     if constexpr (kBrief) {
       if (brief && armed() && (float)st.d <= L.phi_safe && st.a * 2.00002 < L.a_ev)
-        end_ray(2 * nstep - 1);
+        end_ray(TAKEN ? nstep : 2 * nstep - 1);
     }
     if (!__any(armed())) goto done;
     // outbound: u -= du (:274-296)
@@ -667,14 +668,15 @@ __device__ inline void march(const DevScene& s, Lane<float>& L, bool captured, d
 #pragma unroll
       for (int b = 0; b < (NS - 1) / kB; ++b) {
         block(NS + 1 + kB * b, out_coeffs, false, std::integral_constant<int, kB>{});
-        if (beyond(NS + kB * (b + 1))) end_ray(2 * nstep - 1);
+        const int m = NS + kB * (b + 1);
+        if (beyond(m)) end_ray(TAKEN ? m : 2 * nstep - 1);
         if (!__any(armed())) goto done;
       }
       n = NS + 1 + kB * ((NS - 1) / kB);
     } else {
       for (; n + 3 < 2 * nstep; n += 4) {
         block(n, out_coeffs, false, std::integral_constant<int, 4>{});
-        if (beyond(n + 3)) end_ray(2 * nstep - 1);
+        if (beyond(n + 3)) end_ray(TAKEN ? n + 3 : 2 * nstep - 1);
         if (!__any(armed())) goto done;
       }
     }

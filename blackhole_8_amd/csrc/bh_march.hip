@@ -266,6 +266,40 @@ hipError_t launch_turning(const DevScene* scene, double* l, int W, int H, hipStr
   return hipGetLastError();
 }
 
+// The steps that the march of a frame without the swept-angle plane takes of
+// each ray (discs and holes only): 0 where the set-up ends it or leaves it to
+// the FP64 pass.
+template <int NS>
+__global__ __launch_bounds__(256) void steps_taken_kernel(const DevScene* __restrict__ sp,
+                                                          int32_t* __restrict__ taken) {
+  const DevScene& s = *sp;
+  const int x = blockIdx.x * 16 + (threadIdx.x & 15);
+  const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
+  if (x >= s.W || y >= s.H) return;
+  const DevOut out{nullptr, nullptr, nullptr, nullptr, nullptr};
+  RaySetup r;
+  setup_ray32<false, false>(s, out, x, y, r);
+  MarchOut<float> mo;
+  mo.steps = 0;
+  if (!r.degenerate && !r.over && !r.band) {
+    Lane<float> L;
+    const double du = (r.l - s.u0) * s.inv_nstep;
+    setup_lane<float>(s, r.l, r.ib2, du, r.e2x, r.e2y, r.e2z, r.sgn, L);
+    march<false, false, NS, true>(s, L, r.captured, r.first_aa, du, brief_march(out), mo);
+  }
+  taken[(size_t)y * s.W + x] = mo.steps;
+}
+
+hipError_t launch_steps_taken(const DevScene* scene, int32_t* taken, int W, int H, int nstep,
+                              hipStream_t stream) {
+  const dim3 g((W + 15) / 16, (H + 15) / 16);
+  if (nstep == kRefSteps)
+    hipLaunchKernelGGL((steps_taken_kernel<kRefSteps>), g, dim3(256), 0, stream, scene, taken);
+  else
+    hipLaunchKernelGGL((steps_taken_kernel<0>), g, dim3(256), 0, stream, scene, taken);
+  return hipGetLastError();
+}
+
 // FP64 pass of one frame.
 hipError_t launch_band(const DevScene* scene, const DevOut& out, const DevQueue& q,
                        hipStream_t stream, bool escape, bool spheres) {

@@ -31,6 +31,16 @@ Work of a frame = F_SETUP * rays + F_STEP * sum(steps) + F_HIT * hits, plus
 for spheres (F_SPH_RAY + F_SPH_PLANE * spheres) * rays +
 F_SPH_STEP * sum(steps * spheres in the pixel's plane), plus F_BG * escaped
 rays, with the per-pixel step counts and hit classes of the render itself.
+
+The FP32 march of holes and discs ends a ray once nothing is left for it to
+meet (frames without the swept-angle plane).  The work it does (taken_flops)
+charges the steps it takes of each ray (bh_steps_taken), and where it takes
+none, because the set-up ends the ray or leaves it to the FP64 pass,
+
+  F_PIXEL        60  of the set-up: pixel point, orbit-plane frame, b, Y0
+
+alone.  The first count is what the reference's rule would take for the frame;
+over the march's time it is no rate of the hardware.
 """
 from __future__ import annotations
 
@@ -39,6 +49,7 @@ import numpy as np
 F_STEP_DISC = 35
 F_STEP_NODISC = 30
 F_SETUP = 240
+F_PIXEL = 60
 F_HIT = 40
 F_SPH_RAY = 9
 F_SPH_PLANE = 7
@@ -93,3 +104,13 @@ def frame_flops(steps: np.ndarray, hit: np.ndarray, has_disc: bool,
     if background:
         work += F_BG * int((hit == 0).sum())
     return float(work)
+
+
+def taken_flops(taken: np.ndarray, hit: np.ndarray, has_disc: bool) -> float:
+    """Work of one frame's march that ends rays early, from the steps it takes
+    of each ray and the hit classes (no escape, no spheres)."""
+    f_step = F_STEP_DISC if has_disc else F_STEP_NODISC
+    marched = taken > 0
+    n = int(marched.sum())
+    return float(F_SETUP * n + F_PIXEL * (taken.size - n) + f_step * int(taken.sum(dtype=np.int64))
+                 + F_HIT * int(((hit != 0) & marched).sum()))

@@ -106,6 +106,13 @@ class Renderer:
                                             C.byref(m), C.byref(t), C.byref(n)))
         return m.value, t.value, n.value
 
+    def steps_taken(self, scene: abi.Scene, opts: abi.Options) -> np.ndarray:
+        """Steps the FP32 march takes of each ray (bh_steps_taken)."""
+        n = np.empty((scene.camera.height, scene.camera.width), np.int32)
+        self._check(self.lib.bh_steps_taken(self.ctx, C.byref(scene), C.byref(opts),
+                                            n.ctypes.data_as(C.POINTER(C.c_int32))))
+        return n
+
     # -- batches ------------------------------------------------------------
     def render_batch(self, items, want=("rgb", "hit"), tuning: abi.BatchTuning | None = None,
                      timing: bool = False):

@@ -326,6 +326,15 @@ int bh_chord_sincos(bh_ctx* ctx, const float* x_host, float* sc_host, int64_t n)
 int bh_turning_points(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
                       double* l_host);
 
+/* Measurement helper with no counterpart in the reference: the steps that the
+ * FP32 march of a frame without the swept-angle plane takes of each pixel's ray
+ * before nothing is left for it to meet (the steps plane holds those of the
+ * reference's rule); 0 where the ray's set-up ends it or leaves it to the FP64
+ * pass.  Frames in which no ray ends early (FP64 march, escape, spheres):
+ * BH_ERR_UNSUPPORTED.  steps_host receives width x height counts, row-major. */
+int bh_steps_taken(bh_ctx* ctx, const bh_scene* scene, const bh_options* opt,
+                   int32_t* steps_host);
+
 /* ======================================================================== */
 /* Batches: many independent scenes in one persistent launch (no reference  */
 /* counterpart: the reference renders one scene at a time,                  */

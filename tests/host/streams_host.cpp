@@ -252,6 +252,10 @@ hipError_t launch_turning(const DevScene* s, double* l, int, int, hipStream_t st
   launch("turning", st, {s}, {l});
   return hipSuccess;
 }
+hipError_t launch_steps_taken(const DevScene* s, int32_t* n, int, int, int, hipStream_t st) {
+  launch("steps taken", st, {s}, {n});
+  return hipSuccess;
+}
 hipError_t launch_chord_sincos(const float* x, float* o, int, hipStream_t st) {
   launch("sincos", st, {x}, {o});
   return hipSuccess;
